@@ -6,8 +6,10 @@
  * 1-based `cmalloc(n)-1` arrays are passed as `&arr[1]`).  Orbital blocks use
  * the reference's storage: separate real / imaginary FP64 arrays, state-major,
  * `ncoef` coefficients per state with G=0 stored last (entry ncoef-1), Gamma
- * symmetry c(-G) = c(G)*.  The real-space grid is the FFTW (a,b,c) row-major
- * grid with c fastest.
+ * symmetry c(-G) = c(G)*.  Wherever a call takes orbitals (or v_ext) as a re
+ * and an im array it also takes one interleaved complex array z, given as
+ * re = (double *)z, im = (double *)z + 1.  The real-space grid is the FFTW
+ * (a,b,c) row-major grid with c fastest.
  *
  * Every function returns 0 on success and a negative SDFT_E* code on error;
  * sdft_hip_last_error() returns a message for the last error on the calling

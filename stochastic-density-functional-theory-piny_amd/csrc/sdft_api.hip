@@ -258,6 +258,8 @@ static int build_geometry(Ctx& c, const sdft_grid_desc* d) {
   if ((rc = upload(&c.t.coef_plus, coef_plus))) return rc;
   if ((rc = upload(&c.t.coef_minus, coef_minus))) return rc;
   if ((rc = upload(&c.t.ak2, g.ak2))) return rc;
+  if ((rc = upload(&c.t.perm, g.perm))) return rc;
+  if ((rc = upload(&c.t.iperm, g.iperm))) return rc;
   double* t64 = nullptr;
   float* t32 = nullptr;
   if ((rc = upload(&t64, tw64))) return rc;
@@ -267,8 +269,16 @@ static int build_geometry(Ctx& c, const sdft_grid_desc* d) {
   return 0;
 }
 
+static void block_free(Block& b);
+
 static void free_ctx(Ctx& c) {
   rs_free(c);
+  if (c.ws) {
+    block_free(*c.ws);
+    delete c.ws;
+    c.ws = nullptr;
+  }
+  if (c.io_pin) (void)hipHostFree(c.io_pin);
   if (c.dens) {
     free_ctx(*c.dens);
     delete c.dens;
@@ -280,7 +290,7 @@ static void free_ctx(Ctx& c) {
                   c.t.tw32,     c.vks64,        c.vks32,       c.A64,          c.A32,
                   c.At64,       c.At32,
                   c.E,          c.W,            c.W2,          c.zpart,        c.Y,           c.Y32,
-                  c.Z,          c.red};
+                  c.Z,          c.red,          c.t.perm,      c.t.iperm,      c.io_dev,      c.arena};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c.ev_cur) (void)hipEventDestroy(c.ev_cur);
@@ -405,44 +415,298 @@ static void block_free(Block& b) {
   b = Block();
 }
 
-// host (reference order, re/im arrays) -> device internal layout
-static int block_put(Block& b, double* dst, const double* re, const double* im) {
-  Ctx& c = *b.ctx;
-  const int nc = c.g.ncoef, ncp = c.g.ncp;
-  std::vector<double> h((size_t)b.nstate_pad * 2 * ncp, 0.0);
-  for (int s = 0; s < b.nstate; ++s) {
-    double* row = h.data() + (size_t)s * 2 * ncp;
-    const double* r = re + (size_t)s * nc;
-    const double* i = im + (size_t)s * nc;
-    for (int j = 0; j < nc; ++j) {
-      row[j] = r[c.g.perm[j]];
-      row[ncp + j] = i[c.g.perm[j]];
-    }
+// ---- orbital transfers ------------------------------------------------------
+// Orbitals cross the host boundary in the caller's coefficient order: either
+// separate re / im arrays, or one interleaved complex array given as (p, p +
+// 1).  The permutation to the internal order, the padding and the split into
+// re / im halves happen in these kernels, on data copied as it is (or, for
+// small transfers, read from and written to pinned host memory directly: no
+// copy operation on the stream at all).  The host permutation they replace
+// (through a zeroed temporary, then a pageable copy) took 6 ms for 256 Si64
+// orbitals (12.6 MB); the copy alone takes 0.7 ms.
+
+// X[s][j], X[s][ncp + j] = re / im of state s at caller index perm[j]; padding
+// and the states [ns_in, gridDim.y) are zero.  dst2 (nullable) receives the
+// same, dst32 (nullable) the same in float.
+__global__ __launch_bounds__(256) void k_orb_put(const double* __restrict__ re,
+                                                 const double* __restrict__ im, int stride,
+                                                 const int* __restrict__ perm, int ncoef, int ncp,
+                                                 int ns_in, double* __restrict__ dst,
+                                                 double* __restrict__ dst2,
+                                                 float* __restrict__ dst32) {
+  const int j = blockIdx.x * 256 + threadIdx.x, s = blockIdx.y;
+  if (j >= ncp) return;
+  double x = 0.0, y = 0.0;
+  if (j < ncoef && s < ns_in) {
+    const size_t i = ((size_t)s * ncoef + perm[j]) * stride;
+    x = re[i];
+    y = im[i];
   }
-  SDFT_HIP_CHECK(hipMemcpyAsync(dst, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice,
-                                c.stream));
-  SDFT_HIP_CHECK(hipStreamSynchronize(c.stream));
+  const size_t o = (size_t)s * 2 * ncp + j;
+  dst[o] = x;
+  dst[o + ncp] = y;
+  if (dst2) {
+    dst2[o] = x;
+    dst2[o + ncp] = y;
+  }
+  if (dst32) {
+    dst32[o] = float(x);
+    dst32[o + ncp] = float(y);
+  }
+}
+
+// the reverse: caller order, states blockIdx.y
+__global__ __launch_bounds__(256) void k_orb_get(const double* __restrict__ src,
+                                                 const int* __restrict__ iperm, int ncoef, int ncp,
+                                                 int stride, double* __restrict__ re,
+                                                 double* __restrict__ im) {
+  const int i = blockIdx.x * 256 + threadIdx.x, s = blockIdx.y;
+  if (i >= ncoef) return;
+  const size_t o = (size_t)s * 2 * ncp + iperm[i];
+  const size_t d = ((size_t)s * ncoef + i) * stride;
+  re[d] = src[o];
+  im[d] = src[o + ncp];
+}
+
+constexpr size_t kPinUp = 256 * 1024, kPinDown = 512 * 1024;  // bytes of pinned memory
+constexpr size_t kStageBytes = size_t(64) << 20;              // device staging, at most
+
+static int io_pinned(Ctx& c) {
+  if (c.io_pin) return 0;
+  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&c.io_pin), kPinUp + kPinDown,
+                               hipHostMallocDefault);
+  if (e != hipSuccess) {
+    c.io_pin = nullptr;
+    return hip_fail(e, "hipHostMalloc (orbital transfers)", __FILE__, __LINE__);
+  }
   return 0;
 }
 
+static int io_staging(Ctx& c, size_t bytes) {
+  if (c.io_dev_bytes >= bytes) return 0;
+  SDFT_HIP_CHECK(hipStreamSynchronize(c.stream));
+  if (c.io_dev) SDFT_HIP_CHECK(hipFree(c.io_dev));
+  c.io_dev = nullptr;
+  c.io_dev_bytes = 0;
+  int rc = dalloc(&c.io_dev, bytes);
+  if (rc) return rc;
+  c.io_dev_bytes = bytes;
+  return 0;
+}
+
+static bool interleaved(const double* re, const double* im) { return im == re + 1; }
+
+// states per staging pass: as many as the staging buffer may hold, at least one
+static int io_states(int nstate, size_t state_bytes) {
+  const size_t n = std::max<size_t>(1, kStageBytes / state_bytes);
+  return (int)std::min<size_t>(n, (size_t)nstate);
+}
+
+// host orbitals -> device internal layout (queued on the context's stream;
+// the caller's arrays must stay valid until the call's final wait)
+static int block_put(Block& b, double* dst, const double* re, const double* im,
+                     double* dst2 = nullptr, float* dst32 = nullptr) {
+  Ctx& c = *b.ctx;
+  const int nc = c.g.ncoef, ncp = c.g.ncp;
+  const bool il = interleaved(re, im);
+  const size_t per = (size_t)nc * 2 * sizeof(double);  // one state
+  int rc;
+  if (per * b.nstate <= kPinUp) {
+    // the previous call that used the pinned region has waited for its kernels
+    if ((rc = io_pinned(c))) return rc;
+    const size_t half = (size_t)nc * b.nstate;
+    if (il) {
+      memcpy(c.io_pin, re, 2 * half * sizeof(double));
+    } else {
+      memcpy(c.io_pin, re, half * sizeof(double));
+      memcpy(c.io_pin + half, im, half * sizeof(double));
+    }
+    hipLaunchKernelGGL(k_orb_put, dim3((ncp + 255) / 256, b.nstate_pad), dim3(256), 0, c.stream,
+                       c.io_pin, il ? c.io_pin + 1 : c.io_pin + half, il ? 2 : 1, c.t.perm, nc,
+                       ncp, b.nstate, dst, dst2, dst32);
+    SDFT_HIP_CHECK(hipGetLastError());
+    return 0;
+  }
+  const int step = io_states(b.nstate, per);
+  if ((rc = io_staging(c, per * step))) return rc;
+  for (int s0 = 0; s0 < b.nstate; s0 += step) {
+    const int ns = std::min(step, b.nstate - s0);
+    const int rows = s0 + ns == b.nstate ? b.nstate_pad - s0 : ns;
+    const size_t half = (size_t)nc * ns, off = (size_t)nc * s0;
+    if (il) {
+      SDFT_HIP_CHECK(hipMemcpyAsync(c.io_dev, re + 2 * off, 2 * half * sizeof(double),
+                                    hipMemcpyHostToDevice, c.stream));
+    } else {
+      SDFT_HIP_CHECK(hipMemcpyAsync(c.io_dev, re + off, half * sizeof(double),
+                                    hipMemcpyHostToDevice, c.stream));
+      SDFT_HIP_CHECK(hipMemcpyAsync(c.io_dev + half, im + off, half * sizeof(double),
+                                    hipMemcpyHostToDevice, c.stream));
+    }
+    const size_t o = (size_t)s0 * 2 * ncp;
+    hipLaunchKernelGGL(k_orb_put, dim3((ncp + 255) / 256, rows), dim3(256), 0, c.stream, c.io_dev,
+                       il ? c.io_dev + 1 : c.io_dev + half, il ? 2 : 1, c.t.perm, nc, ncp, ns,
+                       dst + o, dst2 ? dst2 + o : nullptr, dst32 ? dst32 + o : nullptr);
+    SDFT_HIP_CHECK(hipGetLastError());
+  }
+  return 0;
+}
+
+// waits for the context's stream and hands over the small downloads
+static int io_finish(Ctx& c) {
+  hipError_t e = hipStreamSynchronize(c.stream);
+  if (e == hipSuccess)
+    for (const Ctx::PinCopy& p : c.pin_out) {
+      if (interleaved(p.re, p.im)) {
+        memcpy(p.re, p.src, 2 * p.count * sizeof(double));
+      } else {
+        memcpy(p.re, p.src, p.count * sizeof(double));
+        memcpy(p.im, p.src + p.count, p.count * sizeof(double));
+      }
+    }
+  c.pin_out.clear();
+  c.pin_used = 0;
+  if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize", __FILE__, __LINE__);
+  return 0;
+}
+
+// device internal layout -> host orbitals (the caller's arrays hold them
+// after the next io_finish)
 static int block_fetch(Block& b, const double* src, double* re, double* im) {
   Ctx& c = *b.ctx;
   const int nc = c.g.ncoef, ncp = c.g.ncp;
-  std::vector<double> h((size_t)b.nstate_pad * 2 * ncp);
-  SDFT_HIP_CHECK(hipMemcpyAsync(h.data(), src, sizeof(double) * h.size(), hipMemcpyDeviceToHost,
-                                c.stream));
-  SDFT_HIP_CHECK(hipStreamSynchronize(c.stream));
-  for (int s = 0; s < b.nstate; ++s) {
-    const double* row = h.data() + (size_t)s * 2 * ncp;
-    double* r = re + (size_t)s * nc;
-    double* i = im + (size_t)s * nc;
-    for (int j = 0; j < nc; ++j) {
-      r[c.g.perm[j]] = row[j];
-      i[c.g.perm[j]] = row[ncp + j];
+  const bool il = interleaved(re, im);
+  const size_t per = (size_t)nc * 2 * sizeof(double);
+  int rc;
+  if (per * b.nstate <= kPinDown) {
+    if ((rc = io_pinned(c))) return rc;
+    if (c.pin_used + per * b.nstate > kPinDown && (rc = io_finish(c))) return rc;
+    const size_t half = (size_t)nc * b.nstate;
+    double* out = c.io_pin + (kPinUp + c.pin_used) / sizeof(double);
+    c.pin_used += per * b.nstate;
+    hipLaunchKernelGGL(k_orb_get, dim3((nc + 255) / 256, b.nstate), dim3(256), 0, c.stream, src,
+                       c.t.iperm, nc, ncp, il ? 2 : 1, out, il ? out + 1 : out + half);
+    SDFT_HIP_CHECK(hipGetLastError());
+    c.pin_out.push_back({out, re, im, half});
+    return 0;
+  }
+  const int step = io_states(b.nstate, per);
+  if ((rc = io_staging(c, per * step))) return rc;
+  for (int s0 = 0; s0 < b.nstate; s0 += step) {
+    const int ns = std::min(step, b.nstate - s0);
+    const size_t half = (size_t)nc * ns, off = (size_t)nc * s0;
+    hipLaunchKernelGGL(k_orb_get, dim3((nc + 255) / 256, ns), dim3(256), 0, c.stream,
+                       src + (size_t)s0 * 2 * ncp, c.t.iperm, nc, ncp, il ? 2 : 1, c.io_dev,
+                       il ? c.io_dev + 1 : c.io_dev + half);
+    SDFT_HIP_CHECK(hipGetLastError());
+    if (il) {
+      SDFT_HIP_CHECK(hipMemcpyAsync(re + 2 * off, c.io_dev, 2 * half * sizeof(double),
+                                    hipMemcpyDeviceToHost, c.stream));
+    } else {
+      SDFT_HIP_CHECK(hipMemcpyAsync(re + off, c.io_dev, half * sizeof(double),
+                                    hipMemcpyDeviceToHost, c.stream));
+      SDFT_HIP_CHECK(hipMemcpyAsync(im + off, c.io_dev + half, half * sizeof(double),
+                                    hipMemcpyDeviceToHost, c.stream));
     }
   }
   return 0;
 }
+
+// The orbital block of one call on host arrays: the context's kept block
+// where it is (or may be made) large enough, else one of the call's own.  Its
+// padding is zero from its allocation on (no kernel writes there); the rows
+// beyond the call's states hold earlier calls' values, which reach no output.
+struct CallBlock {
+  Ctx& c;
+  Block* b = nullptr;
+  bool own = false;
+  bool waited = false;  // the call has waited for the stream
+  explicit CallBlock(Ctx& cc) : c(cc) {}
+  int get(int nstate, int prec) {
+    const int pad = (nstate + 1) / 2 * 2;
+    const size_t rows = (size_t)(pad + 31) / 32 * 32, row = (size_t)2 * c.g.ncp * sizeof(double);
+    const bool keep = rows * row * 6 <= kKeepBytes;
+    int rc;
+    if (!keep) {
+      own = true;
+      b = new Block();
+      return block_alloc(c, nstate, prec, *b);
+    }
+    if (!c.ws || c.ws_pad < pad || (prec == 1 && !c.ws->X32)) {
+      const int want = std::max(nstate, c.ws_pad);
+      const int wp = prec == 1 || (c.ws && c.ws->X32) ? 1 : 0;
+      SDFT_HIP_CHECK(hipStreamSynchronize(c.stream));
+      if (c.ws) block_free(*c.ws);
+      else c.ws = new Block();
+      c.ws_pad = 0;
+      if ((rc = block_alloc(c, want, wp, *c.ws))) {
+        block_free(*c.ws);
+        delete c.ws;
+        c.ws = nullptr;
+        return rc;
+      }
+      c.ws_pad = c.ws->nstate_pad;
+    }
+    b = c.ws;
+    b->nstate = nstate;
+    b->nstate_pad = pad;
+    b->prec = prec;
+    b->cur = 0;
+    return 0;
+  }
+  ~CallBlock() {
+    if (!waited) {
+      (void)hipStreamSynchronize(c.stream);
+      if (c.stream_nl) (void)hipStreamSynchronize(c.stream_nl);
+      c.pin_out.clear();
+      c.pin_used = 0;
+    }
+    if (own && b) {
+      block_free(*b);
+      delete b;
+    }
+  }
+};
+
+// Scratch of one call: the context's arena, or memory of the call's own
+// where it needs more than a context keeps.
+struct CallArena {
+  Ctx& c;
+  char* p = nullptr;
+  size_t used = 0, have = 0;
+  bool own = false;
+  explicit CallArena(Ctx& cc) : c(cc) {}
+  static size_t up(size_t n) { return (n + 255) / 256 * 256; }
+  int reserve(size_t bytes) {
+    have = bytes;
+    if (bytes > kKeepBytes) {
+      own = true;
+      return dalloc(&p, bytes);
+    }
+    if (c.arena_bytes < bytes) {
+      SDFT_HIP_CHECK(hipStreamSynchronize(c.stream));
+      if (c.arena) SDFT_HIP_CHECK(hipFree(c.arena));
+      c.arena = nullptr;
+      c.arena_bytes = 0;
+      int rc = dalloc(&c.arena, bytes);
+      if (rc) return rc;
+      c.arena_bytes = bytes;
+    }
+    p = static_cast<char*>(c.arena);
+    return 0;
+  }
+  template <typename T>
+  T* take(size_t n) {
+    T* r = reinterpret_cast<T*>(p + used);
+    used += up(n * sizeof(T));
+    return r;
+  }
+  ~CallArena() {
+    if (own && p) {
+      (void)hipStreamSynchronize(c.stream);
+      (void)hipFree(p);
+    }
+  }
+};
 
 __global__ void k_to_f32(const double* __restrict__ x, float* __restrict__ y, size_t n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -603,8 +867,9 @@ static int block_noise_impl(Block& b, long long seed, long long first) {
 }
 
 // The Chebyshev filter on resident data (filter.c:318-706).
+// have32: X32 holds T_0 in float (FP32 form)
 static int block_filter_impl(Block& b, int L, const double* coeffs, double scale, double emean,
-                             double* moments) {
+                             double* moments, bool have32 = false) {
   Ctx& c = *b.ctx;
   int rc;
   if ((rc = check_vks(c))) return rc;
@@ -643,7 +908,7 @@ static int block_filter_impl(Block& b, int L, const double* coeffs, double scale
     double* cur = bufs[(k - 1) & 1];
     double* out = bufs[k & 1];
     if ((rc = apply_step(b, kModeFilter, cur, out, sp, moments ? b.mom_part : nullptr,
-                         fuse_flags(c, k, L))))
+                         fuse_flags(c, k, L) | (have32 ? kHaveX32 : 0))))
       return rc;
   }
   // T_{L-1} sits in bufs[(L-1) & 1]
@@ -772,7 +1037,7 @@ static int real_table_impl(Ctx& c) {
       if ((rc = launch_contract(c, 0, kModeNoise, c.W, nq, tmp.X0, tmp.X0, tmp.chi, nullptr,
                                 nullptr, sp, nullptr)))
         break;
-      if ((rc = block_fetch(tmp, tmp.X0, bre.data(), bim.data()))) break;
+      if ((rc = block_fetch(tmp, tmp.X0, bre.data(), bim.data())) || (rc = io_finish(c))) break;
       for (int p = p0; p < p1; ++p) {
         const double* r = bre.data() + (size_t)(p - p0) * c.g.ncoef;
         const double* i = bim.data() + (size_t)(p - p0) * c.g.ncoef;
@@ -832,9 +1097,11 @@ static int nl_forces_real(Ctx& c, int nstate, const double* re, const double* im
       set_error("projector atom index out of range");
       return SDFT_EINVAL;
     }
-  Block b;
-  int rc = block_alloc(c, nstate, 0, b);
-  if (!rc) rc = block_put(b, b.X0, re, im);
+  CallBlock cb(c);
+  int rc = cb.get(nstate, 0);
+  if (rc) return rc;
+  Block& b = *cb.b;
+  rc = block_put(b, b.X0, re, im);
   const int npairs = b.nstate_pad / 2;
   if (!rc) rc = ensure_W(c, w_bytes(c, npairs, 0));
   if (!rc) rc = launch_expand(c, 0, b.X0, npairs, c.W);
@@ -847,8 +1114,8 @@ static int nl_forces_real(Ctx& c, int nstate, const double* re, const double* im
       for (int j = 0; j < 3; ++j)
         forces[proj_atom[p] * 3 + j] +=
             2.0 * energy[p] * vol_elem * S[(size_t)p * 3 + j] / N * occ / nsto;
+    cb.waited = true;  // rs_force_sums
   }
-  block_free(b);
   return rc;
 }
 
@@ -987,45 +1254,43 @@ int sdft_hip_nl_forces(sdft_ctx* h, int nstate, const double* re, const double* 
       set_error("projector atom index out of range");
       return SDFT_EINVAL;
     }
-  Block b;
-  int rc = block_alloc(c, nstate, 0, b);
-  if (!rc) rc = block_put(b, b.X0, re, im);
+  CallBlock cb(c);
+  CallArena ar(c);
+  int rc = cb.get(nstate, 0);
+  if (rc) return rc;
+  Block& b = *cb.b;
   const int ns = b.nstate_pad, ncp = c.g.ncp;
   std::vector<double> gint((size_t)3 * ncp, 0.0);
   for (int j = 0; j < c.g.ncoef; ++j)
     for (int d = 0; d < 3; ++d) gint[(size_t)d * ncp + j] = gvec[(size_t)c.g.perm[j] * 3 + d];
-  double *dg = nullptr, *Ad = nullptr, *Zd = nullptr, *part = nullptr, *S = nullptr;
   int per = 0;
   const int nsplit = kb_project_split(c, ns, &per);
-  if (!rc) rc = upload(&dg, gint);
-  const size_t adbytes = sizeof(double) * (size_t)c.ppad * 2 * ncp;  // zero padding rows
-  if (!rc) rc = dalloc(&Ad, adbytes);
-  if (!rc && hipMemsetAsync(Ad, 0, adbytes, c.stream) != hipSuccess) {
-    set_error("hipMemsetAsync failed");
-    rc = SDFT_EHIP;
-  }
-  if (!rc) rc = dalloc(&Zd, sizeof(double) * (size_t)3 * P * ns);
-  if (!rc) rc = dalloc(&part, sizeof(double) * (size_t)nsplit * P * ns);
-  if (!rc) rc = dalloc(&S, sizeof(double) * (size_t)3 * P);
-  if (!rc) rc = nl_force_sums(c, b.X0, ns, nstate, dg, Ad, Zd, part, S);
+  const size_t ng = gint.size(), nad = (size_t)c.ppad * 2 * ncp, nzd = (size_t)3 * P * ns,
+               npt = (size_t)nsplit * P * ns, nS = (size_t)3 * P;
+  size_t bytes = 0;
+  for (size_t n : {ng, nad, nzd, npt, nS}) bytes += CallArena::up(sizeof(double) * n);
+  if ((rc = ar.reserve(bytes))) return rc;
+  double *dg = ar.take<double>(ng), *Ad = ar.take<double>(nad), *Zd = ar.take<double>(nzd),
+         *part = ar.take<double>(npt), *S = ar.take<double>(nS);
+  if ((rc = block_put(b, b.X0, re, im))) return rc;
   std::vector<double> hs((size_t)3 * P);
-  if (!rc) {
-    hipError_t e = hipMemcpyAsync(hs.data(), S, sizeof(double) * 3 * P, hipMemcpyDeviceToHost,
-                                  c.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
-    if (e != hipSuccess) rc = hip_fail(e, "force download", __FILE__, __LINE__);
-  }
-  if (!rc) {
-    // F_a = -(occ/nsto) sum_{p in a} 2 E_p sum_s Z dZ/dR (calc-nuclei-force.c:462-478 scaling)
-    for (int p = 0; p < P; ++p)
-      for (int d = 0; d < 3; ++d)
-        forces[proj_atom[p] * 3 + d] -= 2.0 * c.E_host[p] * hs[(size_t)p * 3 + d] * occ / nsto;
-  }
-  void* ptrs[] = {dg, Ad, Zd, part, S};
-  for (void* p : ptrs)
-    if (p) (void)hipFree(p);
-  block_free(b);
-  return rc;
+  hipError_t e = hipMemcpyAsync(dg, gint.data(), sizeof(double) * ng, hipMemcpyHostToDevice,
+                                c.stream);
+  // zero padding rows
+  if (e == hipSuccess)
+    e = hipMemsetAsync(Ad + (size_t)P * 2 * ncp, 0, sizeof(double) * (size_t)(c.ppad - P) * 2 * ncp,
+                       c.stream);
+  if (e != hipSuccess) return hip_fail(e, "force upload", __FILE__, __LINE__);
+  if ((rc = nl_force_sums(c, b.X0, ns, nstate, dg, Ad, Zd, part, S))) return rc;
+  e = hipMemcpyAsync(hs.data(), S, sizeof(double) * 3 * P, hipMemcpyDeviceToHost, c.stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+  if (e != hipSuccess) return hip_fail(e, "force download", __FILE__, __LINE__);
+  cb.waited = true;
+  // F_a = -(occ/nsto) sum_{p in a} 2 E_p sum_s Z dZ/dR (calc-nuclei-force.c:462-478 scaling)
+  for (int p = 0; p < P; ++p)
+    for (int d = 0; d < 3; ++d)
+      forces[proj_atom[p] * 3 + d] -= 2.0 * c.E_host[p] * hs[(size_t)p * 3 + d] * occ / nsto;
+  return 0;
 }
 
 int sdft_hip_hpsi(sdft_ctx* h, int nstate, const double* cre, const double* cim, double* fre,
@@ -1037,18 +1302,16 @@ int sdft_hip_hpsi(sdft_ctx* h, int nstate, const double* cre, const double* cim,
   Ctx& c = h->c;
   int rc;
   if ((rc = check_vks(c))) return rc;
-  Block b;
-  if ((rc = block_alloc(c, nstate, prec, b))) {
-    block_free(b);
-    return rc;
-  }
+  CallBlock cb(c);
+  if ((rc = cb.get(nstate, prec))) return rc;
+  Block& b = *cb.b;
   StepParams sp{};
-  if (!(rc = block_put(b, b.X0, cre, cim)) && !(rc = apply_step(b, kModeForce, b.X0, b.X1, sp,
-                                                                  nullptr)))
-    rc = block_fetch(b, b.X1, fre, fim);
-  if (!rc) rc = prof_collect(c);
-  block_free(b);
-  return rc;
+  if ((rc = block_put(b, b.X0, cre, cim, nullptr, b.prec ? b.X32 : nullptr))) return rc;
+  if ((rc = apply_step(b, kModeForce, b.X0, b.X1, sp, nullptr, kHaveX32))) return rc;
+  if ((rc = block_fetch(b, b.X1, fre, fim))) return rc;
+  if ((rc = io_finish(c))) return rc;
+  cb.waited = true;
+  return prof_collect(c);
 }
 
 int sdft_hip_tune(sdft_ctx* h, int nstate, int prec, int steps, int* config_out, int max_cand,
@@ -1176,21 +1439,21 @@ int sdft_hip_newton_filter(sdft_ctx* h, int nstate, int L, int nmu, const double
   Ctx& c = h->c;
   int rc;
   if ((rc = check_vks(c))) return rc;
-  Block b;
-  if ((rc = block_alloc(c, nstate, prec, b))) {
-    block_free(b);
-    return rc;
-  }
+  CallBlock cb(c);
+  CallArena ar(c);
+  if ((rc = cb.get(nstate, prec))) return rc;
+  Block& b = *cb.b;
   const long long stride = (long long)b.nstate_pad * 2 * c.g.ncp;
-  double* accs = nullptr;
-  double* cdev = nullptr;
+  const size_t na = (size_t)stride * nmu, ncf = (size_t)L * nmu;
+  if ((rc = ar.reserve(CallArena::up(sizeof(double) * na) + CallArena::up(sizeof(double) * ncf))))
+    return rc;
+  double* accs = ar.take<double>(na);
+  double* cdev = ar.take<double>(ncf);
   do {
-    if ((rc = dalloc(&accs, sizeof(double) * (size_t)stride * nmu))) break;
-    if ((rc = dalloc(&cdev, sizeof(double) * (size_t)L * nmu))) break;
     SDFT_HIP_TRY(rc, hipMemcpyAsync(cdev, coeffs, sizeof(double) * (size_t)L * nmu,
                                     hipMemcpyHostToDevice, c.stream));
     if (rc) break;
-    if ((rc = block_put(b, b.X0, cre, cim))) break;
+    if ((rc = block_put(b, b.X0, cre, cim, nullptr, b.prec ? b.X32 : nullptr))) break;
     if (L == 1) {
       for (int mu = 0; mu < nmu; ++mu) {
         hipLaunchKernelGGL(k_scale_copy, dim3((unsigned)((stride + 255) / 256)), dim3(256), 0,
@@ -1219,7 +1482,8 @@ int sdft_hip_newton_filter(sdft_ctx* h, int nstate, int L, int nmu, const double
       sp.c0 = 0.0;
       sp.first = (n == 1);
       sp.step = n;
-      rc = apply_step(b, kModeNewton, X[(n - 1) & 1], X[n & 1], sp, nullptr, fuse_flags(c, n, L));
+      rc = apply_step(b, kModeNewton, X[(n - 1) & 1], X[n & 1], sp, nullptr,
+                      fuse_flags(c, n, L) | kHaveX32);
     }
     b.acc = own_acc;
     c.newton_nmu = 0;
@@ -1227,18 +1491,16 @@ int sdft_hip_newton_filter(sdft_ctx* h, int nstate, int L, int nmu, const double
     c.newton_c = nullptr;
     if (rc) break;
     if ((rc = prof_collect(c))) break;
-    const size_t per = (size_t)nstate * c.g.ncoef;
+    const size_t per = (size_t)nstate * c.g.ncoef * (interleaved(out_re, out_im) ? 2 : 1);
     for (int mu = 0; mu < nmu && !rc; ++mu)
       rc = block_fetch(b, accs + (size_t)mu * stride, out_re + mu * per, out_im + mu * per);
     if (!rc) rc = block_fetch(b, X[(L - 1) & 1], cre, cim);
+    if (!rc) rc = io_finish(c);
+    if (!rc) cb.waited = true;
   } while (0);
   c.newton_nmu = 0;
   c.newton_stride = 0;
   c.newton_c = nullptr;
-  void* ptrs[] = {accs, cdev};
-  for (void* p : ptrs)
-    if (p) (void)hipFree(p);
-  block_free(b);
   return rc;
 }
 
@@ -1252,11 +1514,9 @@ int sdft_hip_spectral_bound(sdft_ctx* h, int which, double emax, double conv, in
   Ctx& c = h->c;
   int rc;
   if ((rc = check_vks(c))) return rc;
-  Block b;
-  if ((rc = block_alloc(c, 1, prec, b))) {
-    block_free(b);
-    return rc;
-  }
+  CallBlock cb(c);
+  if ((rc = cb.get(1, prec))) return rc;
+  Block& b = *cb.b;
   // the reference starts from energyOld = 1e7, energy = 1e5 (:168-170) and
   // iterates while |energyOld - energy| > energyConv
   double e_old = 1.0e7, e = 1.0e5;
@@ -1270,9 +1530,10 @@ int sdft_hip_spectral_bound(sdft_ctx* h, int which, double emax, double conv, in
     ++it;
   }
   if (!rc) rc = block_fetch(b, b.X0, vre, vim);
-  if (!rc) rc = prof_collect(c);
-  block_free(b);
+  if (!rc) rc = io_finish(c);
   if (rc) return rc;
+  cb.waited = true;
+  if ((rc = prof_collect(c))) return rc;
   *energy = e;
   if (iters) *iters = it;
   return 0;
@@ -1296,18 +1557,18 @@ int sdft_hip_cheby_filter(sdft_ctx* h, int nstate, int L, const double* coeffs, 
     return SDFT_EINVAL;
   }
   Ctx& c = h->c;
-  Block b;
-  int rc = block_alloc(c, nstate, prec, b);
-  if (!rc) rc = block_put(b, b.X0, cre, cim);
-  if (!rc && moments) {
-    const size_t bytes = sizeof(double) * (size_t)b.nstate_pad * 2 * c.g.ncp;
-    SDFT_HIP_TRY(rc, hipMemcpyAsync(b.chi, b.X0, bytes, hipMemcpyDeviceToDevice, c.stream));
-  }
-  if (!rc) rc = block_filter_impl(b, L, coeffs, scale, emean, moments);
-  if (!rc) rc = block_fetch(b, b.acc, ore, oim);
-  if (!rc) rc = block_fetch(b, b.cur ? b.X1 : b.X0, cre, cim);
-  block_free(b);
-  return rc;
+  CallBlock cb(c);
+  int rc = cb.get(nstate, prec);
+  if (rc) return rc;
+  Block& b = *cb.b;
+  if ((rc = block_put(b, b.X0, cre, cim, moments ? b.chi : nullptr, b.prec ? b.X32 : nullptr)))
+    return rc;
+  if ((rc = block_filter_impl(b, L, coeffs, scale, emean, moments, true))) return rc;
+  if ((rc = block_fetch(b, b.acc, ore, oim))) return rc;
+  if ((rc = block_fetch(b, b.cur ? b.X1 : b.X0, cre, cim))) return rc;
+  if ((rc = io_finish(c))) return rc;
+  cb.waited = true;
+  return 0;
 }
 
 int sdft_hip_cheby_moments(sdft_ctx* h, int nstate, int L, double scale, double emean,
@@ -1319,14 +1580,13 @@ int sdft_hip_cheby_moments(sdft_ctx* h, int nstate, int L, double scale, double 
   Ctx& c = h->c;
   int rc;
   if ((rc = check_vks(c))) return rc;
-  Block b;
-  rc = block_alloc(c, nstate, prec, b);
-  if (!rc) rc = block_put(b, b.X0, cre, cim);
+  CallBlock cb(c);
+  if ((rc = cb.get(nstate, prec))) return rc;
+  Block& b = *cb.b;
+  rc = block_put(b, b.X0, cre, cim, b.chi, b.prec ? b.X32 : nullptr);
   const int nmom = (L % 2 == 0) ? L / 2 + 1 : (L + 1) / 2;
   if (!rc) rc = ensure_mom(b, nmom);
   if (!rc) {
-    const size_t bytes = sizeof(double) * (size_t)b.nstate_pad * 2 * c.g.ncp;
-    SDFT_HIP_TRY(rc, hipMemcpyAsync(b.chi, b.X0, bytes, hipMemcpyDeviceToDevice, c.stream));
     prof_reset(c);
     double* bufs[2] = {b.X0, b.X1};
     for (int k = 1; k < nmom && !rc; ++k) {
@@ -1340,7 +1600,7 @@ int sdft_hip_cheby_moments(sdft_ctx* h, int nstate, int L, double scale, double 
       sp.first = (k == 1);
       sp.step = k;
       rc = apply_step(b, kModeMoments, bufs[(k - 1) & 1], bufs[k & 1], sp, b.mom_part,
-                      fuse_flags(c, k, nmom));
+                      fuse_flags(c, k, nmom) | kHaveX32);
     }
     if (!rc) rc = prof_collect(c);
   }
@@ -1358,9 +1618,9 @@ int sdft_hip_cheby_moments(sdft_ctx* h, int nstate, int L, double scale, double 
         moments[2 * k - 1] = 2.0 * red[3 * k + 1] - moments[1];
         moments[2 * k] = 2.0 * red[3 * k + 2] - moments[0];
       }
+      cb.waited = true;  // moments_reduce
     }
   }
-  block_free(b);
   return rc;
 }
 
@@ -1397,18 +1657,24 @@ int sdft_hip_density(sdft_ctx* h, int nstate, const double* re, const double* im
     return SDFT_EINVAL;
   }
   Ctx& c = h->c;
-  Block b;
-  int rc = block_alloc(c, nstate, 0, b);
-  if (!rc) rc = block_put(b, b.X0, re, im);
+  CallBlock cb(c);
+  CallArena ar(c);
+  int rc = cb.get(nstate, 0);
+  if (rc) return rc;
+  Block& b = *cb.b;
+  rc = block_put(b, b.X0, re, im);
   const int npairs = b.nstate_pad / 2;
   const int ngroups = std::max(1, std::min(npairs, 2048 / c.g.n));
-  double* part = nullptr;
-  double* drho = nullptr;
+  const size_t npart = (size_t)ngroups * c.g.N, nrho = (size_t)c.g.N;
   if (!rc) rc = ensure_W(c, w_bytes(c, npairs, 0));
-  if (!rc) rc = dalloc(&part, sizeof(double) * (size_t)ngroups * c.g.N);
-  if (!rc) rc = dalloc(&drho, sizeof(double) * (size_t)c.g.N);
-  if (!rc && accumulate) {
-    hipError_t e = hipMemcpy(drho, rho, sizeof(double) * c.g.N, hipMemcpyHostToDevice);
+  if (!rc)
+    rc = ar.reserve(CallArena::up(sizeof(double) * npart) + CallArena::up(sizeof(double) * nrho));
+  if (rc) return rc;
+  double* part = ar.take<double>(npart);
+  double* drho = ar.take<double>(nrho);
+  if (accumulate) {
+    hipError_t e = hipMemcpyAsync(drho, rho, sizeof(double) * c.g.N, hipMemcpyHostToDevice,
+                                  c.stream);
     if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy rho", __FILE__, __LINE__);
   }
   if (!rc) rc = launch_expand(c, 0, b.X0, npairs, c.W);
@@ -1419,10 +1685,8 @@ int sdft_hip_density(sdft_ctx* h, int nstate, const double* re, const double* im
                                   c.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
     if (e != hipSuccess) rc = hip_fail(e, "density download", __FILE__, __LINE__);
+    else cb.waited = true;
   }
-  if (part) (void)hipFree(part);
-  if (drho) (void)hipFree(drho);
-  block_free(b);
   return rc;
 }
 
@@ -1433,9 +1697,11 @@ int sdft_hip_energies(sdft_ctx* h, int nstate, const double* re, const double* i
     return SDFT_EINVAL;
   }
   Ctx& c = h->c;
-  Block b;
-  int rc = block_alloc(c, nstate, 0, b);
-  if (!rc) rc = block_put(b, b.X0, re, im);
+  CallBlock cb(c);
+  int rc = cb.get(nstate, 0);
+  if (rc) return rc;
+  Block& b = *cb.b;
+  rc = block_put(b, b.X0, re, im);
   double ke = 0.0, nl = 0.0;
   if (!rc) rc = energy_ke_device(c, b.X0, nstate, &ke);
   if (!rc && rs_active(c)) {
@@ -1453,8 +1719,8 @@ int sdft_hip_energies(sdft_ctx* h, int nstate, const double* re, const double* i
   if (!rc) {
     *eke = occ * 0.5 * ke / nsto;
     *enl = occ * nl / nsto;
+    cb.waited = true;  // the reductions
   }
-  block_free(b);
   return rc;
 }
 
@@ -1489,10 +1755,11 @@ int sdft_hip_block_set(sdft_block* bb, const double* cre, const double* cim) {
   }
   Block& b = bb->b;
   b.cur = 0;
-  int rc = block_put(b, b.X0, cre, cim);
-  if (rc) return rc;
-  const size_t bytes = sizeof(double) * (size_t)b.nstate_pad * 2 * b.ctx->g.ncp;
-  SDFT_HIP_CHECK(hipMemcpyAsync(b.chi, b.X0, bytes, hipMemcpyDeviceToDevice, b.ctx->stream));
+  int rc = block_put(b, b.X0, cre, cim, b.chi);
+  if (rc) {
+    (void)hipStreamSynchronize(b.ctx->stream);
+    return rc;
+  }
   SDFT_HIP_CHECK(hipStreamSynchronize(b.ctx->stream));
   return 0;
 }
@@ -1503,11 +1770,12 @@ int sdft_hip_noise(sdft_ctx* h, int nstate, long long seed, long long first, dou
     set_error("bad noise arguments");
     return SDFT_EINVAL;
   }
-  Block b;
-  int rc = block_alloc(h->c, nstate, 0, b);
-  if (!rc) rc = block_noise_impl(b, seed, first);
-  if (!rc) rc = block_fetch(b, b.X0, cre, cim);
-  block_free(b);
+  CallBlock cb(h->c);
+  int rc = cb.get(nstate, 0);
+  if (!rc) rc = block_noise_impl(*cb.b, seed, first);
+  if (!rc) rc = block_fetch(*cb.b, cb.b->X0, cre, cim);
+  if (!rc) rc = io_finish(h->c);
+  if (!rc) cb.waited = true;
   return rc;
 }
 
@@ -1540,7 +1808,9 @@ int sdft_hip_block_get(sdft_block* bb, int which, double* re, double* im) {
   }
   Block& b = bb->b;
   const double* src = which == 0 ? b.acc : (b.cur ? b.X1 : b.X0);
-  return block_fetch(b, src, re, im);
+  int rc = block_fetch(b, src, re, im);
+  const int rc2 = io_finish(*b.ctx);
+  return rc ? rc : rc2;
 }
 
 int sdft_hip_set_profiling(sdft_ctx* h, int on) {
@@ -1643,9 +1913,10 @@ int sdft_hip_ks_potential(sdft_ctx* h, const double* rho, int layout, const doub
   SDFT_HIP_CHECK(hipMemcpyAsync(c.ks_io, rho, sizeof(double) * N, hipMemcpyHostToDevice, s));
   if ((rc = launch_ks_field(s, c.ks_io, layout, n, N, volume, c.ks_field, c.ks_rho))) return rc;
   if ((rc = ensure_W(dc, w_bytes(dc, 1, 0)))) return rc;
-  Block b;
-  rc = block_alloc(dc, 1, 0, b);
-  if (!rc) rc = launch_grid_plane(dc, dc.W, 1, c.ks_field);
+  CallBlock cb(dc);
+  if ((rc = cb.get(1, 0))) return rc;
+  Block& b = *cb.b;
+  rc = launch_grid_plane(dc, dc.W, 1, c.ks_field);
   StepParams sp{};
   if (!rc)
     rc = launch_contract(dc, 0, kModeNoise, dc.W, 1, b.X0, b.X0, b.chi, nullptr, nullptr, sp,
@@ -1679,7 +1950,7 @@ int sdft_hip_ks_potential(sdft_ctx* h, const double* rho, int layout, const doub
     }
   }
   (void)hipStreamSynchronize(s);
-  block_free(b);
+  cb.waited = true;
   if (rc) return rc;
   c.have_vks = true;
   c.ks_have_q = true;

@@ -77,6 +77,8 @@ struct DeviceTables {
   int* coef_plus = nullptr;   // [ncoef] (d << 8) | ia of +G (internal order)
   int* coef_minus = nullptr;  // [ncoef] (d << 8) | ia of -G
   double* ak2 = nullptr;      // [ncp] internal order
+  int* perm = nullptr;        // [ncoef] internal j -> caller index
+  int* iperm = nullptr;       // [ncoef] caller index -> internal j
   void* tw64 = nullptr;       // [n] double2 exp(+2 pi i m/n)
   void* tw32 = nullptr;       // [n] float2
 };
@@ -89,6 +91,13 @@ constexpr unsigned kSyncEventFlags = hipEventDisableTiming | hipEventDisableSyst
 
 // Per-atom real-space KB data (sdft_hip_set_projectors_real), see sdft_rs.hip.
 struct RsKB;
+struct Block;
+
+// Device memory that a context keeps between calls for the calls' own use
+// (orbital blocks of calls on host arrays, partial sums): per buffer at most
+// this much; a call that needs more allocates for itself and frees at its
+// end.  Everything is released with the context.
+constexpr size_t kKeepBytes = size_t(256) << 20;
 
 struct Ctx {
   int device = 0;
@@ -128,6 +137,23 @@ struct Ctx {
   int Y_ppad = 0;
   double* red = nullptr;     // reduction scratch
   size_t red_bytes = 0;
+  // the orbital block of calls on host arrays, and their scratch arena
+  Block* ws = nullptr;
+  int ws_pad = 0;            // states it holds (padded)
+  void* arena = nullptr;
+  size_t arena_bytes = 0;
+  // transfers of orbitals (block_put / block_fetch): device staging in the
+  // caller's order, and pinned host memory for small ones
+  double* io_dev = nullptr;
+  size_t io_dev_bytes = 0;
+  double* io_pin = nullptr;  // [kPinUp + kPinDown bytes]
+  struct PinCopy {
+    const double* src;
+    double *re, *im;
+    size_t count;  // values per part
+  };
+  std::vector<PinCopy> pin_out;  // downloads to hand over at the next io_finish
+  size_t pin_used = 0;
   // launch configuration (the tuner's pick): plane-kernel tile variant (0
   // base sub-chunk, 1 double) and the KB projection's target workgroup count
   int plane_variant = 0;  // plane-kernel variant, 0 .. plane_variant_count(n) - 1

@@ -3,7 +3,8 @@
 The library must have been built (sdft_amd.build.build()); importing this
 module never falls back to a CPU path: a missing library or a failing call
 raises.  Orbital blocks are numpy complex arrays (nstate, ncoef) with G=0
-last, split into the separate FP64 real / imaginary arrays the C ABI takes.
+last, passed to the C ABI as they are (its interleaved form: the address of
+the first real part and the address one double further).
 """
 from __future__ import annotations
 
@@ -136,9 +137,15 @@ def _check(rc):
         raise SdftError("sdft_hip error %d: %s" % (rc, msg))
 
 
-def _split(Cz):
-    Cz = np.ascontiguousarray(Cz)
-    return np.ascontiguousarray(Cz.real, dtype=np.float64), np.ascontiguousarray(Cz.imag, dtype=np.float64)
+def _orb(Cz):
+    """A contiguous complex128 array of orbitals and its (re, im) addresses."""
+    Cz = np.ascontiguousarray(Cz, dtype=np.complex128)
+    a = Cz.ctypes.data
+    return Cz, C.cast(a, _dp), C.cast(a + 8, _dp)
+
+
+def _new_orb(*shape):
+    return _orb(np.empty(shape, dtype=np.complex128))
 
 
 def selftest_fft(x: np.ndarray, direction: int, prec: int = PREC_FP64) -> np.ndarray:
@@ -227,12 +234,10 @@ class Context:
         _check(self.lib.sdft_hip_set_projectors(self.h, 0, None, None, None))
 
     def hpsi_raw(self, Cz, prec=PREC_FP64):
-        re, im = _split(Cz)
-        fre = np.empty_like(re)
-        fim = np.empty_like(im)
-        _check(self.lib.sdft_hip_hpsi(self.h, re.shape[0], _ptr(re), _ptr(im), _ptr(fre),
-                                      _ptr(fim), prec))
-        return fre + 1j * fim
+        c, re, im = _orb(Cz)
+        f, fre, fim = _new_orb(*c.shape)
+        _check(self.lib.sdft_hip_hpsi(self.h, c.shape[0], re, im, fre, fim, prec))
+        return f
 
     def tune(self, nstate, prec=PREC_FP64, steps=6):
         """sdft_hip_tune: returns ((plane_tile, kb_wg_target, fused_expand),
@@ -262,11 +267,10 @@ class Context:
         if rho.size != self.sys.ngrid or np.size(vext) != len(getattr(self, "_dak2", ())):
             raise SdftError("ks_potential: rho must have n^3 points and vext one value per "
                             "density-sphere coefficient (after ks_init)")
-        vr = np.ascontiguousarray(np.real(vext), dtype=np.float64)
-        vi = np.ascontiguousarray(np.imag(vext), dtype=np.float64)
+        vx, vr, vi = _orb(vext)
         en = np.zeros(4)
         out = np.empty_like(rho)
-        _check(self.lib.sdft_hip_ks_potential(self.h, _ptr(rho), layout, _ptr(vr), _ptr(vi),
+        _check(self.lib.sdft_hip_ks_potential(self.h, _ptr(rho), layout, vr, vi,
                                               float(volume), xc, _ptr(en), _ptr(out)))
         return out, dict(eh=en[0], eext=en[1], exc=en[2], muxc=en[3])
 
@@ -292,30 +296,29 @@ class Context:
     def newton_filter(self, chi, coeffs, samp_point, scale, emean, prec=PREC_FP64):
         """filterNewtonPolyHerm: coeffs (L, nmu), samp_point (L-1,).  Returns
         (out (nmu, nstate, ncoef), P_{L-1})."""
-        re, im = _split(chi)
+        T, re, im = _orb(np.array(chi, dtype=np.complex128))
         co = np.ascontiguousarray(coeffs, dtype=np.float64)
         if co.ndim == 1:
             co = co[:, None]
         L, nmu = co.shape
         z = np.ascontiguousarray(samp_point, dtype=np.float64)
         assert z.shape[0] >= L - 1
-        ns, nc = re.shape
-        ore = np.empty((nmu, ns, nc))
-        oim = np.empty((nmu, ns, nc))
+        ns, nc = T.shape
+        out, ore, oim = _new_orb(nmu, ns, nc)
         _check(self.lib.sdft_hip_newton_filter(self.h, ns, L, nmu, _ptr(co), _ptr(z), scale, emean,
-                                               _ptr(re), _ptr(im), _ptr(ore), _ptr(oim), prec))
-        return ore + 1j * oim, re + 1j * im
+                                               re, im, ore, oim, prec))
+        return out, T
 
     def spectral_bound(self, v0, which, emax=0.0, conv=1e-5, max_iter=100000,
                        prec=PREC_FP64):
         """genEnergyMax (which 0) / genEnergyMin (which 1) on the device from
         the start vector v0 (ncoef complex): returns (E, final vector, iterations)."""
-        re, im = _split(np.asarray(v0).reshape(1, -1))
+        v, re, im = _orb(np.array(v0, dtype=np.complex128).reshape(1, -1))
         e = C.c_double()
         it = C.c_int()
-        _check(self.lib.sdft_hip_spectral_bound(self.h, which, emax, conv, max_iter, _ptr(re),
-                                                _ptr(im), C.byref(e), C.byref(it), prec))
-        return e.value, (re + 1j * im)[0], it.value
+        _check(self.lib.sdft_hip_spectral_bound(self.h, which, emax, conv, max_iter, re,
+                                                im, C.byref(e), C.byref(it), prec))
+        return e.value, v[0], it.value
 
     def cheby_coeffs(self, L, emin, emax, mu, beta, fun_flag=2):
         c = np.empty(L)
@@ -323,22 +326,19 @@ class Context:
         return c
 
     def cheby_filter(self, chi, coeffs, scale, emean, prec=PREC_FP64, moments=False):
-        re, im = _split(chi)
-        ore = np.empty_like(re)
-        oim = np.empty_like(im)
+        T, re, im = _orb(np.array(chi, dtype=np.complex128))
+        out, ore, oim = _new_orb(*T.shape)
         coeffs = np.ascontiguousarray(coeffs, dtype=np.float64)
         mom = np.zeros(len(coeffs)) if moments else None
-        _check(self.lib.sdft_hip_cheby_filter(self.h, re.shape[0], len(coeffs), _ptr(coeffs),
-                                              scale, emean, _ptr(re), _ptr(im), _ptr(ore),
-                                              _ptr(oim), _ptr(mom), prec))
-        out = (ore + 1j * oim, re + 1j * im)
-        return out + (mom,) if moments else out
+        _check(self.lib.sdft_hip_cheby_filter(self.h, T.shape[0], len(coeffs), _ptr(coeffs),
+                                              scale, emean, re, im, ore, oim, _ptr(mom), prec))
+        return (out, T, mom) if moments else (out, T)
 
     def cheby_moments(self, chi, L, scale, emean, prec=PREC_FP64):
-        re, im = _split(chi)
+        c, re, im = _orb(chi)
         mom = np.zeros(L + 1)
-        _check(self.lib.sdft_hip_cheby_moments(self.h, re.shape[0], L, scale, emean, _ptr(re),
-                                               _ptr(im), _ptr(mom), prec))
+        _check(self.lib.sdft_hip_cheby_moments(self.h, c.shape[0], L, scale, emean, re, im,
+                                               _ptr(mom), prec))
         return mom
 
     def chem_pot(self, L, emin, emax, beta, moments, nsto, ne_true, mu_init, gap, occ=2.0,
@@ -354,43 +354,41 @@ class Context:
     def density(self, Cz, occ_over_nsto, layout=RHO_FFTW, accumulate_into=None):
         """rho in FFTW or generic order; with accumulate_into (an FP64 array of
         ngrid) the density is added to it in place and it is returned."""
-        re, im = _split(Cz)
+        c, re, im = _orb(Cz)
         if accumulate_into is None:
             rho = np.zeros(self.sys.ngrid)
         else:
             rho = accumulate_into
             assert rho.dtype == np.float64 and rho.flags.c_contiguous and rho.size == self.sys.ngrid
-        _check(self.lib.sdft_hip_density(self.h, re.shape[0], _ptr(re), _ptr(im), occ_over_nsto,
+        _check(self.lib.sdft_hip_density(self.h, c.shape[0], re, im, occ_over_nsto,
                                          _ptr(rho), layout, 0 if accumulate_into is None else 1))
         return rho
 
     def energies(self, Cz, occ, nsto):
-        re, im = _split(Cz)
+        c, re, im = _orb(Cz)
         eke = C.c_double()
         enl = C.c_double()
-        _check(self.lib.sdft_hip_energies(self.h, re.shape[0], _ptr(re), _ptr(im), occ, nsto,
+        _check(self.lib.sdft_hip_energies(self.h, c.shape[0], re, im, occ, nsto,
                                           C.byref(eke), C.byref(enl)))
         return eke.value, enl.value
 
     def noise(self, nstate, seed, first=0):
         """Stochastic orbitals generated on the device (genNoiseOrbitalReal)."""
-        nc = self.sys.ncoef
-        re = np.empty((nstate, nc))
-        im = np.empty((nstate, nc))
-        _check(self.lib.sdft_hip_noise(self.h, nstate, seed, first, _ptr(re), _ptr(im)))
-        return re + 1j * im
+        out, re, im = _new_orb(nstate, self.sys.ncoef)
+        _check(self.lib.sdft_hip_noise(self.h, nstate, seed, first, re, im))
+        return out
 
     def nl_forces(self, Cz, occ, nsto):
         """Hellmann-Feynman nonlocal forces (natm, 3) of the orbitals Cz."""
         s = self.sys
-        re, im = _split(Cz)
+        c, re, im = _orb(Cz)
         g = np.ascontiguousarray(s.gvec, dtype=np.float64)
         # the atom of each projector the context holds: the real-space ones
         # when set, else the system's G-space table
         pa = self._rs_atom if getattr(self, "_rs_atom", None) is not None else \
             np.ascontiguousarray(s.proj_atom, dtype=np.int32)
         out = np.zeros((s.natm, 3))
-        _check(self.lib.sdft_hip_nl_forces(self.h, re.shape[0], _ptr(re), _ptr(im), _ptr(g),
+        _check(self.lib.sdft_hip_nl_forces(self.h, c.shape[0], re, im, _ptr(g),
                                            pa.ctypes.data_as(_ip), s.natm, occ, nsto, _ptr(out)))
         return out
 
@@ -429,8 +427,8 @@ class Block:
             pass
 
     def set(self, chi):
-        re, im = _split(chi)
-        _check(self.ctx.lib.sdft_hip_block_set(self.h, _ptr(re), _ptr(im)))
+        c, re, im = _orb(chi)
+        _check(self.ctx.lib.sdft_hip_block_set(self.h, re, im))
 
     def noise(self, seed, first=0):
         _check(self.ctx.lib.sdft_hip_block_noise(self.h, seed, first))
@@ -443,11 +441,9 @@ class Block:
         return mom
 
     def get(self, which=0):
-        ncoef = self.ctx.sys.ncoef
-        re = np.empty((self.nstate, ncoef))
-        im = np.empty((self.nstate, ncoef))
-        _check(self.ctx.lib.sdft_hip_block_get(self.h, which, _ptr(re), _ptr(im)))
-        return re + 1j * im
+        out, re, im = _new_orb(self.nstate, self.ctx.sys.ncoef)
+        _check(self.ctx.lib.sdft_hip_block_get(self.h, which, re, im))
+        return out
 
 
 class Batch:
