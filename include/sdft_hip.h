@@ -193,8 +193,8 @@ int sdft_hip_chem_pot(sdft_ctx *ctx, int L, double emin, double emax, double bet
  * memory (code under HIP graph capture, tight serving loops such as the mu
  * search inside an SCF step, harnesses that forbid hipMalloc): the same
  * search as sdft_hip_chem_pot, same arguments, results and errors, but its
- * scratch (cosine table, h_j, moments, result: 2 roundFFT(32 L) + L + 4
- * doubles) lives in a fixed per-device array of 4.3 MB that the library
+ * scratch (unit roots, partial DFT sums, h_j, moments: 4.5 roundFFT(32 L) + L
+ * doubles and a few KB) lives in a fixed per-device array of 10.2 MB that the library
  * holds from load to process end, and the call allocates nothing.  L must
  * not exceed 8192 (SDFT_EINVAL beyond).  All calls on one device share that
  * array: calls that overlap on one device (several host threads, or several
