@@ -743,16 +743,18 @@ static int apply_step(Block& b, int mode, const double* cur, double* out, const 
                        b.X32, n);
     SDFT_HIP_CHECK(hipGetLastError());
   }
-  // The KB chain runs on its own stream, overlapping the FFT kernels; with
-  // profiling on, each kernel's events are recorded on the stream it runs on.
-  const bool overlap = table;
+  // The KB chain overlaps the FFT kernels.  It follows the previous contract on
+  // that kernel's own stream; the FFT kernels and this step's contract go to
+  // the other one, which then is the context's stream (the two swap roles
+  // every step).  So the chain's projection starts first and has its
+  // workgroups placed before the plane kernel fills the chip: started behind
+  // it (5 us later, the time of an event between streams), it got its slots
+  // only as the plane drained and took 63 us instead of 20 (Si64 FP32).
+  // With profiling on, each kernel's events are recorded on the stream it
+  // runs on.
   if (table) {
-    hipStream_t main = c.stream;
-    if (overlap) {
-      SDFT_HIP_CHECK(hipEventRecord(c.ev_cur, c.stream));
-      SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream_nl, c.ev_cur, 0));
-      c.stream = c.stream_nl;
-    }
+    SDFT_HIP_CHECK(hipEventRecord(c.ev_cur, c.stream));
+    SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream_nl, c.ev_cur, 0));
     {
       ProfScope ps(c, "kb_project");
       rc = launch_nl_project(c, b.prec, x32 ? (const void*)b.X32 : (const void*)cur,
@@ -762,11 +764,9 @@ static int apply_step(Block& b, int mode, const double* cur, double* out, const 
       ProfScope ps(c, "kb_force");
       rc = launch_nl_force(c, b.prec, b.nstate_pad, b.fnl);
     }
-    if (overlap) {
-      c.stream = main;
-      SDFT_HIP_CHECK(hipEventRecord(c.ev_nl, c.stream_nl));
-    }
     if (rc) return rc;
+    SDFT_HIP_CHECK(hipEventRecord(c.ev_nl, c.stream));
+    std::swap(c.stream, c.stream_nl);
     fnl = b.fnl;
   }
   if (!(flags & kHaveW)) {
@@ -795,7 +795,7 @@ static int apply_step(Block& b, int mode, const double* cur, double* out, const 
     ProfScope ps(c, "plane_bc_vpsi");
     if ((rc = launch_plane(c, b.prec, c.W, npairs, &Wres))) return rc;
   }
-  if (overlap) SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream, c.ev_nl, 0));
+  if (table) SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream, c.ev_nl, 0));
   {
     ProfScope ps(c, "contract_a");
     if ((rc = launch_contract(c, b.prec, mode, Wres, npairs, cur, out, b.acc, fnl, b.chi, sp,

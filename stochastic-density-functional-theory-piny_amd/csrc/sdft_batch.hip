@@ -79,6 +79,7 @@ struct Group {
   size_t lds = 0;    // plane kernel dynamic LDS, tile variant 0
   size_t lds1 = 0;   // tile variant 1 (0 when it does not fit)
   bool prune = true;  // every fragment's sphere inside |k| < n/4 (pruned plane passes)
+  size_t ldsw = 0;    // wave-private plane stage's LDS (0: it does not apply)
   int tot_exp = 0, tot_plane = 0;
   int* pre_exp = nullptr;    // expand and contract share the (chunk, pair) tiling
   int* pre_plane = nullptr;
@@ -375,6 +376,12 @@ int enqueue_step(Batch& B, int variant, int slot) {
                              g.tot_exp, 0, 0, s)))
         return rc;
   for (Group& g : B.groups) {
+    if (B.plane_variant == 0 && g.ldsw > 0) {
+      if ((rc = launch_wplane_batch(g.n, B.prec, g.plane, g.pre_plane, (int)g.frags.size(),
+                                    g.tot_plane, g.ldsw, s)))
+        return rc;
+      continue;
+    }
     const int v = (B.plane_variant == 1 && g.lds1 > 0) ? 1 : 0;
     if ((rc = launch_batch(1, g.n, B.prec, g.plane, g.pre_plane, (int)g.frags.size(),
                            g.tot_plane, v ? g.lds1 : g.lds, v | (g.prune ? 2 : 0), s)))
@@ -600,7 +607,8 @@ int sdft_hip_batch_create(int nfrag, sdft_block* const* blocks, sdft_batch** out
   if ((rc = upload_vec(B.copy, ca, B.stream))) return fail(rc);
   for (Group& g : B.groups) {
     std::vector<int> pe{0}, pp{0};
-    size_t lds = 0, lds1 = 0;
+    size_t lds = 0, lds1 = 0, ldsw = 0;
+    bool wave = true;
     for (int fi : g.frags) {
       const Frag& f = B.frags[fi];
       pe.push_back(pe.back() + f.c->g.nchunk * f.npairs);
@@ -608,11 +616,15 @@ int sdft_hip_batch_create(int nfrag, sdft_block* const* blocks, sdft_batch** out
       lds = std::max(lds, plane_lds_for(g.n, prec, f.c->g.M, 0));
       lds1 = std::max(lds1, plane_lds_for(g.n, prec, f.c->g.M, 1));
       if (!plane_prunable(f.c->g.K, g.n)) g.prune = false;
+      ldsw = std::max(ldsw, wplane_lds_for(g.n, prec, f.c->g.M));
+      if (!wplane_applies(*f.c, prec, 0)) wave = false;
     }
+    if (!wave) ldsw = 0;
     if (lds > 160 * 1024) {
       set_error("plane buffer exceeds LDS for a fragment grid in this precision");
       return fail(SDFT_EINVAL);
     }
+    g.ldsw = ldsw;
     g.lds = lds;
     g.lds1 = lds1 <= 160 * 1024 ? lds1 : 0;
     g.tot_exp = pe.back();

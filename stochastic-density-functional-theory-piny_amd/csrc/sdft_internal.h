@@ -401,6 +401,27 @@ size_t plane_lds_for(int n, int prec, int M, int variant);
 // the plane kernel's pruned first / last passes need the sphere inside
 // |k| < n/4 on every axis
 inline bool plane_prunable(int K, int n) { return 4 * K < n; }
+// wave-private plane stage (sdft_wplane.hip), spheres inside |k| < n/4: its
+// dynamic LDS (0: grid size not built), its launch (mode 0 fused, 1 to the
+// grid a.field, 2 from it) and its launch over the fragments of a batch
+size_t wplane_lds_for(int n, int prec, int M);
+// Whether a stage of `mode` takes it: wherever it is built, fits LDS and was
+// measured faster.  That is the whole stage at every size (sdft_plane_wave.h),
+// and of the halves to and from the grid (us, mode 2 / mode 1, this stage
+// against the workgroup-wide one, 256 orbitals at 48 and 64, 64 at 128)
+//   FP64  48: 44.5 / 42.2 against 49.4 / 51.0    96: 146 / 118 against 167 / 121
+//         64: 126 / 102 against 126 / 119       128: 311 / 267 against 330 / 277
+//   FP32  48: 27.0 / 25.2 against 34.6 / 32.3    96: 68.5 / 56.6 against 59.0 / 55.0
+//         64: 64.6 / 58.7 against 60.0 / 57.4   128: 196 / 158 against 156 / 140
+// all but the FP32 ones above 48: a half has less arithmetic per grid byte, and
+// there more waves in flight count for more than fewer barriers.
+inline bool wplane_applies(const Ctx& c, int prec, int mode) {
+  return plane_prunable(c.g.K, c.g.n) && wplane_lds_for(c.g.n, prec, c.g.M) > 0 &&
+         !(mode != 0 && prec == 1 && c.g.n > 48);
+}
+int launch_wplane(Ctx& c, int prec, const PlaneArgs& a, int npairs, int mode);
+int launch_wplane_batch(int n, int prec, const void* args, const int* prefix, int nfrag,
+                        int total, size_t lds, hipStream_t s);
 // one launch of kind 0 (expand), 1 (plane; variant bit 0 the tile, bit 1
 // the pruned passes) or 2 (contract; variant 1: with the fused expand) over
 // the fragments whose

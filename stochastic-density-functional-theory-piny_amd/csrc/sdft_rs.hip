@@ -749,6 +749,11 @@ static int plane_field(Ctx& c, int prec, void* W, int npairs) {
     set_error("internal error: real-space grid not produced before its forward transform");
     return SDFT_EINVAL_CODE;
   }
+  if (wplane_applies(c, prec, MODE)) {
+    PlaneArgs a = make_plane_args(c, prec, W);
+    a.field = r.F;
+    return launch_wplane(c, prec, a, npairs, MODE);
+  }
   if (prec == 0) {
     SDFT_SIZE_SWITCH(c.g.n, return (plane_field_impl<double, NN, MODE>(c, W, r.F, npairs)));
   } else {
