@@ -743,7 +743,9 @@ static int apply_step(Block& b, int mode, const double* cur, double* out, const 
                        b.X32, n);
     SDFT_HIP_CHECK(hipGetLastError());
   }
-  // The KB chain overlaps the FFT kernels.  It follows the previous contract on
+  const bool small = table && kb_small_applies(c, b.prec, b.nstate_pad);
+  const void* kbx = x32 ? (const void*)b.X32 : (const void*)cur;
+  // Else the KB chain overlaps the FFT kernels.  It follows the previous contract on
   // that kernel's own stream; the FFT kernels and this step's contract go to
   // the other one, which then is the context's stream (the two swap roles
   // every step).  So the chain's projection starts first and has its
@@ -752,13 +754,12 @@ static int apply_step(Block& b, int mode, const double* cur, double* out, const 
   // only as the plane drained and took 63 us instead of 20 (Si64 FP32).
   // With profiling on, each kernel's events are recorded on the stream it
   // runs on.
-  if (table) {
+  if (table && !small) {
     SDFT_HIP_CHECK(hipEventRecord(c.ev_cur, c.stream));
     SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream_nl, c.ev_cur, 0));
     {
       ProfScope ps(c, "kb_project");
-      rc = launch_nl_project(c, b.prec, x32 ? (const void*)b.X32 : (const void*)cur,
-                             b.nstate_pad);
+      rc = launch_nl_project(c, b.prec, kbx, b.nstate_pad);
     }
     if (!rc) {
       ProfScope ps(c, "kb_force");
@@ -791,11 +792,26 @@ static int apply_step(Block& b, int mode, const double* cur, double* out, const 
       ProfScope ps(c, "plane_r_to_bc");
       if ((rc = rs_from_grid(c, b.prec, c.W, npairs))) return rc;
     }
+  } else if (small) {
+    int nsplit = 0;
+    {
+      ProfScope ps(c, "plane_bc_vpsi");
+      if ((rc = launch_plane_project(c, b.prec, c.W, npairs, kbx, b.nstate_pad, &nsplit)))
+        return rc;
+    }
+    ProfScope ps(c, "kb_force");
+    if (kb_small_fused(c, b.nstate_pad)) {
+      if ((rc = launch_kb_reduce_force(c, b.prec, b.nstate_pad, nsplit, b.fnl))) return rc;
+    } else {
+      if ((rc = launch_nl_reduce(c, b.prec, b.nstate_pad, nsplit))) return rc;
+      if ((rc = launch_nl_force(c, b.prec, b.nstate_pad, b.fnl))) return rc;
+    }
+    fnl = b.fnl;
   } else {
     ProfScope ps(c, "plane_bc_vpsi");
     if ((rc = launch_plane(c, b.prec, c.W, npairs, &Wres))) return rc;
   }
-  if (table) SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream, c.ev_nl, 0));
+  if (table && !small) SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream, c.ev_nl, 0));
   {
     ProfScope ps(c, "contract_a");
     if ((rc = launch_contract(c, b.prec, mode, Wres, npairs, cur, out, b.acc, fnl, b.chi, sp,

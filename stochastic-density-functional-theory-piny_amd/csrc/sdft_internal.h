@@ -419,6 +419,34 @@ inline bool wplane_applies(const Ctx& c, int prec, int mode) {
   return plane_prunable(c.g.K, c.g.n) && wplane_lds_for(c.g.n, prec, c.g.M) > 0 &&
          !(mode != 0 && prec == 1 && c.g.n > 48);
 }
+// Small systems: the KB projection in the plane stage's launch, the reduction
+// and the force product behind it on the same stream.  Against the chain on a
+// second stream this saves the two joins (5-10 us each) and up to three
+// launches a step, and costs the time of the force product, which nothing
+// covers; so it is taken while that product is small: at most kKbSmallFlops
+// operations in FP64, three times that in FP32.  us per filter step, second
+// stream -> one, by grid and states (operations of the force product):
+//   FP64  24, 64: 45 -> 31 (7e6)       FP32  48,  64: 53 -> 51 (1.3e8)
+//         36, 64: 51 -> 45 (4.2e7)           64,  93: 70 -> 65 (3.0e8)
+//         48, 64: 74 -> 69 (1.3e8)           48, 256: 95 -> 95 (5.4e8)
+//         64, 64: 72 -> 76 (2.0e8)           64, 200: 108 -> 110 (7.1e8)
+// The force product sums the partials itself (kb_reduce_force, one launch
+// less) while its tile of 32 states has at most kKbFusedTile projections: each
+// of its workgroups repeats that sum.  Then the projection has at most
+// kKbFusedPartials partials a tile; else one launch reduces them for all, and
+// 128 workgroups of the projection (256: 41.6 against 38.5 us at 36, 17 states) keep them
+// few.  17 states at 24 (64 projections each): 25 us fused, 30 not; at 36 (128):
+// 46 fused, 38 not.
+constexpr double kKbSmallFlops = 1.4e8;
+constexpr int kKbFusedTile = 2048;
+constexpr int kKbFusedPartials = 8192;
+bool kb_small_applies(const Ctx& c, int prec, int ns);
+bool kb_small_fused(const Ctx& c, int ns);
+int launch_nl_reduce(Ctx& c, int prec, int ns, int nsplit);
+int launch_plane_project(Ctx& c, int prec, void* W, int npairs, const void* X, int ns,
+                         int* nsplit);
+int launch_kb_reduce_force(Ctx& c, int prec, int ns, int nsplit, void* fnl);
+int ensure_zpart(Ctx& c, size_t n);
 int launch_wplane(Ctx& c, int prec, const PlaneArgs& a, int npairs, int mode);
 int launch_wplane_batch(int n, int prec, const void* args, const int* prefix, int nfrag,
                         int total, size_t lds, hipStream_t s);
