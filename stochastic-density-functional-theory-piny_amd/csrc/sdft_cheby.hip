@@ -303,11 +303,21 @@ __global__ void k_enl(const double* __restrict__ Z, const double* __restrict__ E
 // (stodft/calc-spectral-range.c:180-221 / :380-420) on orbital 0 of X with
 // raw force F: h = -f/4 (G != 0), -f/2 (G = 0); E = 2 sum_{G!=0} (h.re v.re +
 // h.im v.im) + h.re(0) v.re(0); w = h (mode 0) or emax v - h (mode 1);
-// v = w / sqrt(2 sum_{G!=0} |w|^2 + w.re(0)^2).  out[0] = E.  One workgroup.
+// v = w / sqrt(2 sum_{G!=0} |w|^2 + w.re(0)^2).  One workgroup.
+// The loop's state lives here, so that the next iteration is in the queue
+// before the host has seen this one: st = {E of the iteration before, E,
+// iterations}; an update after |st[0] - st[1]| <= conv changes nothing.
+// `seen` (pinned host memory) receives a copy of st.
 __global__ void k_power_update(double* __restrict__ X, const double* __restrict__ F, int ncp,
-                               int ncoef, int mode, double emax, double* __restrict__ out) {
+                               int ncoef, int mode, double emax, double conv,
+                               double* __restrict__ st, double* __restrict__ seen) {
   __shared__ double sh[16];
   __shared__ double len_sh;
+  const double e1 = st[1];
+  if (!(fabs(st[0] - e1) > conv)) {
+    if (threadIdx.x < 3) seen[threadIdx.x] = st[threadIdx.x];
+    return;
+  }
   double e = 0.0, l2 = 0.0;
   const int g0 = ncoef - 1;
   for (int j = threadIdx.x; j < ncoef; j += blockDim.x) {
@@ -329,7 +339,9 @@ __global__ void k_power_update(double* __restrict__ X, const double* __restrict_
   e = block_sum(e, sh);
   l2 = block_sum(l2, sh);
   if (threadIdx.x == 0) {
-    out[0] = e;
+    seen[0] = st[0] = e1;
+    seen[1] = st[1] = e;
+    seen[2] = st[2] = st[2] + 1.0;
     len_sh = sqrt(l2);
   }
   __syncthreads();
@@ -340,15 +352,21 @@ __global__ void k_power_update(double* __restrict__ X, const double* __restrict_
   }
 }
 
-// v /= sqrt(<v|v>) (Gamma norm) for orbital 0 of X
-__global__ void k_normalize0(double* __restrict__ X, int ncp, int ncoef) {
+// v /= sqrt(<v|v>) (Gamma norm) for orbital 0 of X; the power iteration's state
+// starts from energyOld = 1e7, energy = 1e5 (calc-spectral-range.c:168-170)
+__global__ void k_normalize0(double* __restrict__ X, int ncp, int ncoef, double* __restrict__ st) {
   __shared__ double sh[16];
   __shared__ double len_sh;
   double l2 = 0.0;
   for (int j = threadIdx.x; j < ncoef; j += blockDim.x)
     l2 += (j == ncoef - 1) ? X[j] * X[j] : 2.0 * (X[j] * X[j] + X[ncp + j] * X[ncp + j]);
   l2 = block_sum(l2, sh);
-  if (threadIdx.x == 0) len_sh = sqrt(l2);
+  if (threadIdx.x == 0) {
+    len_sh = sqrt(l2);
+    st[0] = 1.0e7;
+    st[1] = 1.0e5;
+    st[2] = 0.0;
+  }
   __syncthreads();
   const double inv = 1.0 / len_sh;
   for (int j = threadIdx.x; j < ncoef; j += blockDim.x) {
@@ -562,22 +580,19 @@ int energy_ke_device(Ctx& c, const double* X, int nstate, double* out) {
   return 0;
 }
 
-int normalize0_device(Ctx& c, double* X) {
-  hipLaunchKernelGGL(k_normalize0, dim3(1), dim3(1024), 0, c.stream, X, c.g.ncp, c.g.ncoef);
+int power_start_device(Ctx& c, double* X) {
+  int rc = ensure_red(c, 3 * sizeof(double));
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_normalize0, dim3(1), dim3(1024), 0, c.stream, X, c.g.ncp, c.g.ncoef, c.red);
   SDFT_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
-int power_update_device(Ctx& c, double* X, const double* F, int mode, double emax,
-                        double* energy_host) {
-  int rc = ensure_red(c, sizeof(double));
-  if (rc) return rc;
+int power_update_device(Ctx& c, double* X, const double* F, int mode, double emax, double conv,
+                        double* seen) {
   hipLaunchKernelGGL(k_power_update, dim3(1), dim3(1024), 0, c.stream, X, F, c.g.ncp, c.g.ncoef,
-                     mode, emax, c.red);
+                     mode, emax, conv, c.red, seen);
   SDFT_HIP_CHECK(hipGetLastError());
-  SDFT_HIP_CHECK(hipMemcpyAsync(energy_host, c.red, sizeof(double), hipMemcpyDeviceToHost,
-                                c.stream));
-  SDFT_HIP_CHECK(hipStreamSynchronize(c.stream));
   return 0;
 }
 

@@ -108,6 +108,7 @@ struct Ctx {
   hipStream_t stream_nl = nullptr;
   hipEvent_t ev_cur = nullptr;
   hipEvent_t ev_nl = nullptr;
+  hipEvent_t ev_it[2] = {nullptr, nullptr};  // spectral bound: iterations in flight
   Geometry g;
   DeviceTables t;
   double* vks64 = nullptr;   // [N]
@@ -510,9 +511,9 @@ int chem_pot_device_noalloc(Ctx& c, int L, double emin, double emax, double beta
 int moments_reduce(Ctx& c, const double* mom_part, int nsteps, int nwg, double* out3);
 int energy_ke_device(Ctx& c, const double* X, int nstate, double* out);
 int energy_nl_device(Ctx& c, int nstate_pad, int nstate, double* out);
-int normalize0_device(Ctx& c, double* X);
-int power_update_device(Ctx& c, double* X, const double* F, int mode, double emax,
-                        double* energy_host);
+int power_start_device(Ctx& c, double* X);
+int power_update_device(Ctx& c, double* X, const double* F, int mode, double emax, double conv,
+                        double* seen);
 
 }  // namespace sdft
 
