@@ -466,6 +466,61 @@ SDFT_DEVI void fft_passes_io(Cx<T>* buf, int ld, int nlines, const Cx<T>* tw, in
   }
 }
 
+// Real multipliers vf(line, pos) of the outputs of a last pass, loaded ahead of
+// it (a last pass's outputs lie where its inputs do: j + r N / R).
+template <typename T, int N, int MAXLINES, int NT, bool LINE_FAST, int S, class VF>
+SDFT_DEVI void fft_last_mul_load(
+    int nlines, int tid, VF& vf,
+    T (&mv)[PassShape<T, N, n_passes(N, S) - 1, false, MAXLINES, NT, S>::MAXB]
+           [PassShape<T, N, n_passes(N, S) - 1, false, MAXLINES, NT, S>::R]) {
+  using Sh = PassShape<T, N, n_passes(N, S) - 1, false, MAXLINES, NT, S>;
+  const int total = nlines * Sh::NB;
+  const float rn = slot_rcp(nlines);
+#pragma unroll
+  for (int b = 0; b < Sh::MAXB; ++b) {
+    const int idx = tid + b * NT;
+    int line = 0, j = 0;
+    if (idx < total) slot_map<LINE_FAST, Sh::NB>(idx, nlines, rn, line, j);
+#pragma unroll
+    for (int r = 0; r < Sh::R; ++r) mv[b][r] = vf(line, j + r * Sh::NB);
+  }
+}
+
+// The last pass of an inverse transform with those multipliers where
+// mk(line, pos) holds.
+template <typename T, int N, int MAXLINES, int NT, bool LINE_FAST, int S, class LF, class MK,
+          class SF>
+SDFT_DEVI void fft_last_pass_mul(
+    int nlines, const Cx<T>* tw, int tid, LF& lf,
+    T (&mv)[PassShape<T, N, n_passes(N, S) - 1, false, MAXLINES, NT, S>::MAXB]
+           [PassShape<T, N, n_passes(N, S) - 1, false, MAXLINES, NT, S>::R],
+    MK& mk, SF& sf) {
+  constexpr int P = n_passes(N, S) - 1;
+  using Sh = PassShape<T, N, P, false, MAXLINES, NT, S>;
+  const int total = nlines * Sh::NB;
+  const float rn = slot_rcp(nlines);
+  typename Sh::Regs v;
+  fft_pass_load<T, N, P, false, MAXLINES, NT, LINE_FAST, false, S>(nlines, tid, lf, v);
+#pragma unroll
+  for (int b = 0; b < Sh::MAXB; ++b) {
+    const int idx = tid + b * NT;
+    if (idx < total) {
+      int line, j;
+      slot_map<LINE_FAST, Sh::NB>(idx, nlines, rn, line, j);
+#pragma unroll
+      for (int r = 1; r < Sh::R; ++r) v[b][r] = cmul(v[b][r], tw[mul24(r, j)]);
+      Dft<T, Sh::R, +1>::run(v[b]);
+#pragma unroll
+      for (int r = 0; r < Sh::R; ++r) {
+        const int pos = j + r * Sh::NB;
+        const T m = mk(line, pos) ? mv[b][r] : T(1);
+        sf(line, pos, cx(m * v[b][r].x, m * v[b][r].y));
+      }
+    }
+  }
+  __syncthreads();
+}
+
 // Last pass of an inverse transform (standard order), a real multiplier
 // vf(line, pos) at every output position, and the first pass of the forward
 // transform in reversed order, in registers.  Outputs land at j*R + r.

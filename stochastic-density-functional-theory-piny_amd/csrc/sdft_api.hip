@@ -780,7 +780,7 @@ static int apply_step(Block& b, int mode, const double* cur, double* out, const 
   if (rs) {
     {
       ProfScope ps(c, "plane_bc_to_r");
-      if ((rc = rs_to_grid(c, b.prec, c.W, npairs))) return rc;
+      if ((rc = rs_to_grid(c, b.prec, c.W, npairs, true))) return rc;
     }
     {
       ProfScope ps(c, "rs_project");
@@ -1123,7 +1123,7 @@ static int nl_forces_real(Ctx& c, int nstate, const double* re, const double* im
   const int npairs = b.nstate_pad / 2;
   if (!rc) rc = ensure_W(c, w_bytes(c, npairs, 0));
   if (!rc) rc = launch_expand(c, 0, b.X0, npairs, c.W);
-  if (!rc) rc = rs_to_grid(c, 0, c.W, npairs);
+  if (!rc) rc = rs_to_grid(c, 0, c.W, npairs, false);
   std::vector<double> S((size_t)nproj * 3);
   if (!rc) rc = rs_force_sums(c, npairs, S.data());
   if (!rc) {
@@ -1747,7 +1747,7 @@ int sdft_hip_energies(sdft_ctx* h, int nstate, const double* re, const double* i
     const int npairs = b.nstate_pad / 2;
     rc = ensure_W(c, w_bytes(c, npairs, 0));
     if (!rc) rc = launch_expand(c, 0, b.X0, npairs, c.W);
-    if (!rc) rc = rs_to_grid(c, 0, c.W, npairs);
+    if (!rc) rc = rs_to_grid(c, 0, c.W, npairs, false);
     if (!rc) rc = rs_project(c, 0, npairs);
     if (!rc) rc = rs_energy(c, npairs, nstate, &nl);
   } else if (!rc && c.nproj > 0) {

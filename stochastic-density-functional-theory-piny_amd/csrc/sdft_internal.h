@@ -245,6 +245,8 @@ struct PlaneArgs {
   int M;
   const void* v;
   const void* tw;
+  // real-space KB path: tiles it leaves alone (bit rb / 16 of [ra][rc / 16]; or null)
+  const unsigned short* skip;
   int gx;  // = n (a-planes); gy = pairs
 };
 
@@ -403,7 +405,7 @@ size_t plane_lds_for(int n, int prec, int M, int variant);
 // |k| < n/4 on every axis
 inline bool plane_prunable(int K, int n) { return 4 * K < n; }
 // wave-private plane stage (sdft_wplane.hip), spheres inside |k| < n/4: its
-// dynamic LDS (0: grid size not built), its launch (mode 0 fused, 1 to the
+// dynamic LDS (0: grid size not built), its launch (mode 0 fused, 1 / 3 to the
 // grid a.field, 2 from it) and its launch over the fragments of a batch
 size_t wplane_lds_for(int n, int prec, int M);
 // Whether a stage of `mode` takes it: wherever it is built, fits LDS and was
@@ -484,7 +486,7 @@ void rs_host_lists(const Ctx& c, int* nproj, const long long** off, const int** 
 // the four stages of the per-atom form on npairs pairs (W in: the a-expansion;
 // W out: what the plane kernel would have produced), and the NL energy sum
 // sum_p E_p dV |Z_p|^2 / N over the pairs' orbitals
-int rs_to_grid(Ctx& c, int prec, void* W, int npairs);
+int rs_to_grid(Ctx& c, int prec, void* W, int npairs, bool with_v);
 int rs_project(Ctx& c, int prec, int npairs);
 int rs_apply(Ctx& c, int prec, int npairs);
 int rs_from_grid(Ctx& c, int prec, void* W, int npairs);

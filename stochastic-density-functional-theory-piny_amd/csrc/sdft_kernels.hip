@@ -681,6 +681,7 @@ PlaneArgs make_plane_args(const Ctx& c, int prec, void* W) {
   a.W = W;
   a.Wout = nullptr;
   a.field = nullptr;
+  a.skip = nullptr;
   a.ncolp = c.g.ncolp;
   a.rowcol = c.t.rowcol;
   a.M = c.g.M;

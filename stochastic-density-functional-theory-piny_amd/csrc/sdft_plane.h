@@ -97,7 +97,10 @@ size_t plane2_lds_bytes(int M) {
 
 // MODE 0: the fused stage (inverse c, inverse b, v.psi, forward b, forward
 // c).  MODE 1 stops at real space: the inverse b-lines are stored to the pair
-// grid a.field[q][ra][rb][rc] (FFTW order).  MODE 2 starts there: the forward
+// grid a.field[q][ra][rb][rc] (FFTW order); MODE 3 is MODE 1 with the points of
+// the 16 x 16 tiles that a.skip marks (bit rb / 16 of skip[ra][rc / 16])
+// already multiplied by v_KS, which is loaded ahead of the line's passes.  MODE 2
+// starts there: the forward
 // b-lines are read from a.field (which already holds v.psi plus the real-space
 // KB term) and the stage continues as MODE 0.
 // SC / SB: the radix schedules (fft_lds.h) of the c-lines and the b-lines.
@@ -151,6 +154,7 @@ __device__ __forceinline__ void plane_body(const PlaneArgs& a, int ra, int q) {
 
   // along b, CB columns rc at a time
   const T* vplane = v + (size_t)ra * N * N;
+  const unsigned short* skip = a.skip + (MODE == 3 ? ra * (N / 16) : 0);
   for (int rc0 = 0; rc0 < N; rc0 += CB) {
     auto lp = [&](int l, int pos) {
       const int kb = pos <= N / 2 ? pos : pos - N;
@@ -165,12 +169,22 @@ __device__ __forceinline__ void plane_body(const PlaneArgs& a, int ra, int q) {
       const int kb = pos <= N / 2 ? pos : pos - N;
       if (kb >= -K && kb <= K) Pl[(kb + K) * LDC + lds_slot<PAD>(rc0 + l)] = x;
     };
-    if constexpr (MODE == 1) {
+    if constexpr (MODE == 1 || MODE == 3) {
       // inverse b-lines straight to the real-space grid (consecutive threads
       // on consecutive lines: runs of CB consecutive rc)
       auto sf = [&](int l, int pos, Cx<T> x) { F[(size_t)pos * N + rc0 + l] = x; };
-      fft_passes_io<T, N, +1, false, 0, P - 1, CB, NT, true, PR, false, false, SB, true, true>(
-          Q, LD, CB, tw, tid, lp, sf);
+      if constexpr (MODE == 3) {
+        auto mk = [&](int l, int pos) { return (skip[(rc0 + l) >> 4] >> (pos >> 4)) & 1; };
+        using PL = PassShape<T, N, P - 1, false, CB, NT, SB>;
+        T mv[PL::MAXB][PL::R];
+        fft_last_mul_load<T, N, CB, NT, true, SB>(CB, tid, vf, mv);
+        fft_passes_io<T, N, +1, false, 0, P - 2, CB, NT, true, PR, false, false, SB, true, false>(
+            Q, LD, CB, tw, tid, lp, sq);
+        fft_last_pass_mul<T, N, CB, NT, true, SB>(CB, tw, tid, lq, mv, mk, sf);
+      } else {
+        fft_passes_io<T, N, +1, false, 0, P - 1, CB, NT, true, PR, false, false, SB, true, true>(
+            Q, LD, CB, tw, tid, lp, sf);
+      }
     } else if constexpr (MODE == 2) {
       auto lf = [&](int l, int pos) { return F[(size_t)pos * N + rc0 + l]; };
       fft_passes_io<T, N, -1, true, 0, P - 1, CB, NT, true, false, PR, false, SB, true, true>(
@@ -191,7 +205,7 @@ __device__ __forceinline__ void plane_body(const PlaneArgs& a, int ra, int q) {
   }
 
   // forward along c: LDS -> W
-  if constexpr (MODE != 1)
+  if constexpr (MODE != 1 && MODE != 3)
   for (int r0 = 0; r0 < M; r0 += ML) {
     const int nl = M - r0 < ML ? M - r0 : ML;
     const int* rc = rowcol + (size_t)r0 * N;
@@ -238,7 +252,7 @@ size_t plane_split_lds_bytes(int M) {
   return sizeof(Cx<T>) * ((size_t)M * C::LDH + (size_t)(PADQ ? C::QEP : C::QE) + N);
 }
 
-// MODE 1 / 2 as in plane_body: per half, the inverse b-lines go to the
+// MODE 1 / 2 / 3 as in plane_body: per half, the inverse b-lines go to the
 // real-space grid a.field (no forward part), or the forward b-lines come from
 // it (no inverse part; W is not read, the output goes to Wout).
 template <typename T, int N, int MODE = 0, int NT = kThreads, int V = 0>
@@ -265,6 +279,7 @@ __device__ __forceinline__ void plane_split_body(const PlaneArgs& a, int ra, int
   const Cx<T>* Wp = W + ((size_t)q * N + ra) * ncolp;
   Cx<T>* Wq = Wo + ((size_t)q * N + ra) * ncolp;
   const T* vplane = v + (size_t)ra * N * N;
+  const unsigned short* skip = a.skip + (MODE == 3 ? ra * (N / 16) : 0);
   const Cx<T> zero = cx(T(0), T(0));
   Cx<T>* __restrict__ F = reinterpret_cast<Cx<T>*>(a.field) + ((size_t)q * N + ra) * N * N;
   for (int h = 0; h < 2; ++h) {
@@ -316,10 +331,22 @@ __device__ __forceinline__ void plane_split_body(const PlaneArgs& a, int ra, int
       // use) and the half's rows are read by the first pass only (modes 0 /
       // 1) or written by the last pass only (mode 2): the passes that read or
       // write outside Q skip the barrier between their loads and stores
-      if constexpr (MODE == 1) {
+      if constexpr (MODE == 1 || MODE == 3) {
         auto sf = [&](int l, int pos, Cx<T> x) { F[(size_t)pos * N + c_lo + rc0 + l] = x; };
-        fft_passes_io<T, N, +1, false, 0, P - 1, CB, NT, true, false, false, false, 0, true,
-                      true>(Q, LD, nb, tw, tid, lp, sf);
+        if constexpr (MODE == 3) {
+          auto mk = [&](int l, int pos) {
+            return (skip[(c_lo + rc0 + l) >> 4] >> (pos >> 4)) & 1;
+          };
+          using PL = PassShape<T, N, P - 1, false, CB, NT>;
+          T mv[PL::MAXB][PL::R];
+          fft_last_mul_load<T, N, CB, NT, true, 0>(nb, tid, vf, mv);
+          fft_passes_io<T, N, +1, false, 0, P - 2, CB, NT, true, false, false, false, 0, true,
+                        false>(Q, LD, nb, tw, tid, lp, sq);
+          fft_last_pass_mul<T, N, CB, NT, true, 0>(nb, tw, tid, lq, mv, mk, sf);
+        } else {
+          fft_passes_io<T, N, +1, false, 0, P - 1, CB, NT, true, false, false, false, 0, true,
+                        true>(Q, LD, nb, tw, tid, lp, sf);
+        }
       } else if constexpr (MODE == 2) {
         fft_pass_finish<T, N, -1, 0, true, CB, NT, true>(nb, tw, tid, fpre, sq);
         if (rc0 + CB < H) {
@@ -340,7 +367,7 @@ __device__ __forceinline__ void plane_split_body(const PlaneArgs& a, int ra, int
       }
     }
     // forward along c of the rows with the other half zero: store / add
-    if constexpr (MODE != 1)
+    if constexpr (MODE != 1 && MODE != 3)
     for (int r0 = 0; r0 < M; r0 += ML) {
       const int nl = M - r0 < ML ? M - r0 : ML;
       const int* rc = rowcol + (size_t)r0 * N;

@@ -342,8 +342,9 @@ __device__ __forceinline__ void wplane_body(const PlaneArgs& a, int ra, int q) {
     WTwiddle<T, B> ti;
     WTwiddle<T, FB> tf;
     if constexpr (MODE != 2) ti.load(tw, lane);
-    if constexpr (MODE != 1) tf.load(tw, lane);
+    if constexpr (MODE == 0 || MODE == 2) tf.load(tw, lane);
     const T* vplane = reinterpret_cast<const T*>(a.v) + (size_t)ra * N * N;
+    const unsigned short* skip = a.skip + (MODE == 3 ? ra * (N / 16) : 0);
     for (int c0 = wave * L; c0 < N; c0 += NW * L) {
       Cx<T> u[B::MAXB][B::R];
       if constexpr (MODE == 2) {
@@ -357,7 +358,7 @@ __device__ __forceinline__ void wplane_body(const PlaneArgs& a, int ra, int q) {
       } else {
         // v_KS of this lane's points, in flight during the transform
         T sv[B::MAXB][B::R];
-        if constexpr (MODE == 0) {
+        if constexpr (MODE == 0 || MODE == 3) {
 #pragma unroll
           for (int b = 0; b < B::MAXB; ++b) {
             const int ii = B::live(lane + 64 * b) ? lane + 64 * b : 0;
@@ -384,11 +385,20 @@ __device__ __forceinline__ void wplane_body(const PlaneArgs& a, int ra, int q) {
         wfirst<T, A, +1, true>(v);
         wexchange<T, A, B, S::LDB>(Q, lane, v, u);
         wsecond<T, B, +1>(ti, u);
-        if constexpr (MODE == 1) {
+        if constexpr (MODE == 1 || MODE == 3) {
 #pragma unroll
           for (int b = 0; b < B::MAXB; ++b) {
             const int idx = lane + 64 * b;
             if (B::live(idx)) {
+              if constexpr (MODE == 3) {  // v_KS where its tile is marked (plane_body)
+                const int marks = skip[(c0 + B::line(idx)) >> 4];
+#pragma unroll
+                for (int r = 0; r < B::R; ++r) {
+                  const int rb = B::bfly(idx) + r * B::NB;
+                  const T m = (marks >> (rb >> 4)) & 1 ? sv[b][r] : T(1);
+                  u[b][r] = cx(m * u[b][r].x, m * u[b][r].y);
+                }
+              }
               Cx<T>* dst = F + (size_t)B::bfly(idx) * N + c0 + B::line(idx);
 #pragma unroll
               for (int r = 0; r < B::R; ++r) dst[(size_t)r * B::NB * N] = u[b][r];
@@ -402,7 +412,7 @@ __device__ __forceinline__ void wplane_body(const PlaneArgs& a, int ra, int q) {
               u[b][r] = cx(u[b][r].x * sv[b][r], u[b][r].y * sv[b][r]);
         }
       }
-      if constexpr (MODE != 1) {
+      if constexpr (MODE == 0 || MODE == 2) {
         Cx<T> w[FB::MAXB][FB::R];
         wfirst<T, FA, -1, false>(u);
         wexchange<T, FA, FB, S::LDB>(Q, lane, u, w);
@@ -426,7 +436,7 @@ __device__ __forceinline__ void wplane_body(const PlaneArgs& a, int ra, int q) {
   }
 
   // forward along c: rows of the plane -> W
-  if constexpr (MODE != 1) {
+  if constexpr (MODE == 0 || MODE == 2) {
     __syncthreads();
     using A = WPass<N, false, true, LC, false>;
     using B = WPass<N, true, true, LC, false>;

@@ -12,7 +12,9 @@
 //                [K_a x pairs] product per atom (the channels of an atom
 //                share its point list, gridNlppMap);
 //   rs_apply     k_rs_apply: z(r) <- v(r) z(r) + sum_p w_p(r) Z_p(pair) with
-//                w_p = E_p vol_elem beta_p, at every grid point through the
+//                w_p = E_p vol_elem beta_p, at every grid point (where much of
+//                the cell is vacuum: of every tile with a projector's point,
+//                the others get their v(r) in rs_to_grid) through the
 //                point -> projector inverse lists -- the daxpy into
 //                forceTemp and the scatter-add of :404-441 plus z v (:78, :97);
 //   rs_from_grid (plane stage, MODE 2): forward b and c transforms back to W.
@@ -48,6 +50,14 @@ constexpr int kRsMaxSlots = 256;
 constexpr size_t kRsStageBytes = 64 * 1024;
 constexpr int kRsRegEntries = 8;
 constexpr int kRsAccPairs = 8;
+// Tiles without a projector entry (vacuum) are left to the plane stage, which
+// multiplies them by v on the way to the grid (MODE 3), and the apply kernel
+// neither reads nor writes them -- where they are at least one in
+// kRsSkipShare of all tiles.  A slab at 192^3, 32 orbitals in FP64 (two tiles
+// in three empty): apply 825 -> 291 us, to-grid 773 -> 739 us with v_KS loaded
+// ahead of each line's passes (992 us with v_KS loaded where it is used).  In
+// a full cell nothing is empty and the stage stays as it is.
+constexpr int kRsSkipShare = 8;
 
 // grid point of thread t of apply block b.  Tiled: blocks of kRsApplyPoints
 // points, tb x tc in (rb, rc) with tc the run along rc (tb = points / tc),
@@ -85,6 +95,11 @@ struct RsKB {
   int* bpoff = nullptr;       // [nblock + 1]
   int* bpp = nullptr;         // projector ids
   int nblock = 0;
+  // blocks with at least one entry, where the others are worth leaving out (else
+  // null: all blocks); skip: the others as PlaneArgs takes them
+  int* blist = nullptr;
+  unsigned short* skip = nullptr;
+  int ncover = 0;
   int max_slots = 0;          // largest staged set
   bool tiled = false;         // (rb, rc) tiles of 256 points (else runs of 256 points)
   int tile_c = 0;             // the tiles' extent along rc (0: runs)
@@ -146,7 +161,7 @@ static int rs_grow(void** p, size_t* have, size_t need) {
 
 static void rs_release(RsKB* r) {
   void* ptrs[] = {r->goff,   r->gidx,  r->gval64, r->gval32, r->gp0,   r->gnch,
-                  r->ptoff,  r->ptslot, r->ptw64, r->ptw32, r->bpoff, r->bpp,
+                  r->ptoff,  r->ptslot, r->ptw64, r->ptw32, r->bpoff, r->bpp,   r->blist, r->skip,
                   r->escale, r->F,     r->Z,     r->epart,  r->gdev,  r->fpart};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -332,6 +347,18 @@ int rs_set(Ctx& c, int nproj, const long long* off, const int* idx, const double
     bpp.insert(bpp.end(), set.begin(), set.end());
     bpoff.push_back((int)bpp.size());
   }
+  std::vector<int> blist;
+  const int nt = n / kRsTile;
+  std::vector<unsigned short> skip((size_t)(tiled ? n * nt : 0), 0);
+  for (int b = 0; b < nblock; ++b)
+    if (bpoff[(size_t)b + 1] > bpoff[(size_t)b]) {
+      blist.push_back(b);
+    } else if (tiled) {  // block (ra, rb tile, rc tile)
+      const int ra = b / (nt * nt), ib = b / nt % nt, ic = b % nt;
+      skip[(size_t)ra * nt + ic] |= (unsigned short)(1 << ib);
+    }
+  r->ncover = (int)blist.size();
+  const bool leave = tiled && nblock - r->ncover >= nblock / kRsSkipShare;
   r->tiled = tiled;
   r->tile_c = tc;
   r->nblock = nblock;
@@ -351,6 +378,8 @@ int rs_set(Ctx& c, int nproj, const long long* off, const int* idx, const double
   if (!rc) rc = rs_upload(&r->ptslot, ptslot, c.stream);
   if (!rc) rc = rs_upload(&r->bpoff, bpoff, c.stream);
   if (!rc) rc = rs_upload(&r->bpp, bpp, c.stream);
+  if (!rc && leave) rc = rs_upload(&r->blist, blist, c.stream);
+  if (!rc && leave) rc = rs_upload(&r->skip, skip, c.stream);
   if (!rc) rc = rs_upload(&r->ptw64, ptw, c.stream);
   if (!rc) rc = rs_upload(&r->ptw32, ptw32, c.stream);
   if (!rc) rc = rs_upload(&r->escale, esc, c.stream);
@@ -489,13 +518,14 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_project(
 template <typename T, int QA = kRsAccPairs, int ER = kRsRegEntries>
 __global__ __launch_bounds__(kRsThreads) void k_rs_apply(
     const long long* __restrict__ ptoff, const int* __restrict__ ptslot, const T* __restrict__ ptw,
-    const int* __restrict__ bpoff, const int* __restrict__ bpp, const T* __restrict__ v,
+    const int* __restrict__ blist, const int* __restrict__ bpoff, const int* __restrict__ bpp,
+    const T* __restrict__ v,
     const Cx<T>* __restrict__ Z, long long Ngrid, int n, int tc, int npairs, int qz,
     Cx<T>* __restrict__ F) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Cx<T>* Zl = reinterpret_cast<Cx<T>*>(smem_raw);  // [slots][qz + 1]
   const int ldz = qz + 1;
-  const int b = blockIdx.x;
+  const int b = blist ? blist[blockIdx.x] : blockIdx.x;
   const long long r = rs_block_point(b, threadIdx.x, n, tc);
   const bool live = r < Ngrid;
   const int s0 = bpoff[b], ns = bpoff[b + 1] - s0;
@@ -708,10 +738,11 @@ static int launch_plane_split_field(Ctx& c, const PlaneArgs& a, size_t lds, int 
 // the split form (column halves, c-transforms recomputed per half) with 256
 // or 512 threads.
 template <typename T, int N, int MODE>
-static int plane_field_impl(Ctx& c, void* W, void* F, int npairs) {
+static int plane_field_impl(Ctx& c, void* W, const RsKB& r, int npairs) {
   const Geometry& g = c.g;
   PlaneArgs a = make_plane_args(c, prec_of<T>(), W);
-  a.field = F;
+  a.field = r.F;
+  a.skip = r.skip;
   constexpr size_t kLds = 160 * 1024;
   auto waves = [&](size_t lds, int nt) { return lds <= kLds ? (int)(kLds / lds) * (nt / 64) : 0; };
   const size_t l0 = plane2_lds_bytes<T, N, 0>(g.M), l1 = plane2_lds_bytes<T, N, 1>(g.M);
@@ -742,7 +773,7 @@ static int plane_field(Ctx& c, int prec, void* W, int npairs) {
   RsKB& r = *c.rs;
   const size_t need = (prec == 0 ? sizeof(Cx<double>) : sizeof(Cx<float>)) * (size_t)npairs *
                       (size_t)c.g.N;
-  if (MODE == 1) {
+  if (MODE != 2) {
     int rc = rs_grow(&r.F, &r.F_bytes, need);
     if (rc) return rc;
   } else if (r.F_bytes < need) {
@@ -752,17 +783,21 @@ static int plane_field(Ctx& c, int prec, void* W, int npairs) {
   if (wplane_applies(c, prec, MODE)) {
     PlaneArgs a = make_plane_args(c, prec, W);
     a.field = r.F;
+    a.skip = r.skip;
     return launch_wplane(c, prec, a, npairs, MODE);
   }
   if (prec == 0) {
-    SDFT_SIZE_SWITCH(c.g.n, return (plane_field_impl<double, NN, MODE>(c, W, r.F, npairs)));
+    SDFT_SIZE_SWITCH(c.g.n, return (plane_field_impl<double, NN, MODE>(c, W, r, npairs)));
   } else {
-    SDFT_SIZE_SWITCH(c.g.n, return (plane_field_impl<float, NN, MODE>(c, W, r.F, npairs)));
+    SDFT_SIZE_SWITCH(c.g.n, return (plane_field_impl<float, NN, MODE>(c, W, r, npairs)));
   }
   return 0;
 }
 
-int rs_to_grid(Ctx& c, int prec, void* W, int npairs) { return plane_field<1>(c, prec, W, npairs); }
+// with_v: v(r) z(r) in the tiles that rs_apply will leave out (v_KS is set)
+int rs_to_grid(Ctx& c, int prec, void* W, int npairs, bool with_v) {
+  return with_v && c.rs->skip ? plane_field<3>(c, prec, W, npairs) : plane_field<1>(c, prec, W, npairs);
+}
 
 int rs_from_grid(Ctx& c, int prec, void* W, int npairs) {
   return plane_field<2>(c, prec, W, npairs);
@@ -814,8 +849,10 @@ static int apply_launch(Ctx& c, int npairs, size_t stage_bytes) {
   auto kern = &k_rs_apply<T, QA, ER>;
   SDFT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(kern, dim3(r.nblock), dim3(kRsThreads), lds, c.stream, r.ptoff, r.ptslot,
-                     ptw, r.bpoff, r.bpp, v, reinterpret_cast<const Cx<T>*>(r.Z), N, c.g.n,
+  const int nb = r.blist ? r.ncover : r.nblock;
+  if (nb == 0) return 0;
+  hipLaunchKernelGGL(kern, dim3(nb), dim3(kRsThreads), lds, c.stream, r.ptoff, r.ptslot, ptw,
+                     r.blist, r.bpoff, r.bpp, v, reinterpret_cast<const Cx<T>*>(r.Z), N, c.g.n,
                      r.tile_c, npairs, qz, reinterpret_cast<Cx<T>*>(r.F));
   SDFT_HIP_CHECK(hipGetLastError());
   return 0;

@@ -79,6 +79,14 @@ static int wplane_launch(Ctx& c, const PlaneArgs& a, int npairs) {
 int launch_wplane(Ctx& c, int prec, const PlaneArgs& a, int npairs, int mode) {
   if (mode == 1)
     return prec == 0 ? wplane_launch<double, 1>(c, a, npairs) : wplane_launch<float, 1>(c, a, npairs);
+  if (mode == 3) {
+    // runs of 256 points instead of tiles at 24 and 36: never marked
+    if (c.g.n % 16 != 0) {
+      set_error("internal error: tile marks at a grid without tiles");
+      return SDFT_EINVAL_CODE;
+    }
+    return prec == 0 ? wplane_launch<double, 3>(c, a, npairs) : wplane_launch<float, 3>(c, a, npairs);
+  }
   if (mode == 2)
     return prec == 0 ? wplane_launch<double, 2>(c, a, npairs) : wplane_launch<float, 2>(c, a, npairs);
   return prec == 0 ? wplane_launch<double, 0>(c, a, npairs) : wplane_launch<float, 0>(c, a, npairs);
