@@ -253,6 +253,14 @@ __global__ __launch_bounds__(kThreads) void k_noise_plane(Cx<double>* __restrict
 // ---- K3: forward FFT along a + unpack + force / recurrence ---------------
 // E = true compiles the fused expand (a.Wnext); E = false leaves it out, so
 // the kernel without it keeps its lower register count.
+// A workgroup is one short chain (columns in, transform, update, transform,
+// columns out), so what it costs is memory latency: the chunk's loads are all
+// in flight together, and the update's operands are loaded before the
+// transform (106-122 VGPRs instead of 80-88).  us per launch before -> after:
+// 128^3 FP32, 64 orbitals 74.0 -> 58.8; 24 fragments at 32-48 in FP32
+// 142.7 -> 118.4 (three launches); 32^3 FP64, 64 orbitals 10.9 -> 9.8; at
+// 64^3, 256 orbitals, where it is near the memory's rate (180 MB), 31.3 -> 30.9
+// in FP32 and 37.9 -> 38.2 in FP64.
 template <typename T, int N, bool E>
 __device__ __forceinline__ void contract_body(const ContractArgs& a, int chunk, int q) {
   constexpr int CH = Cfg<N>::CH, LD = Cfg<N>::LD, ML = Cfg<N>::ML;
@@ -303,11 +311,53 @@ __device__ __forceinline__ void contract_body(const ContractArgs& a, int chunk, 
   for (int i = tid; i < N; i += kThreads) tw[i] = twg[i];
   const Cx<T>* Wq = W + (size_t)q * N * ncolp;
   const float rnc = slot_rcp(nc);
-  for (int e = tid; e < nc * N; e += kThreads) {
-    int dl, ra;
-    slot_map<true, 1>(e, nc, rnc, dl, ra);
-    buf[dl * LD + ra] = Wq[(size_t)ra * ncolp + c0 + dl];
+  {
+    // all loads of the chunk in flight before the first is stored
+    constexpr int ME = (CH * N + kThreads - 1) / kThreads;
+    Cx<T> wv[ME];
+    int slot[ME];
+#pragma unroll
+    for (int i = 0; i < ME; ++i) {
+      const int e = tid + i * kThreads;
+      int dl, ra;
+      slot_map<true, 1>(e < nc * N ? e : 0, nc, rnc, dl, ra);
+      wv[i] = Wq[(size_t)ra * ncolp + c0 + dl];
+      slot[i] = dl * LD + ra;
+    }
+#pragma unroll
+    for (int i = 0; i < ME; ++i)
+      if (tid + i * kThreads < nc * N) buf[slot[i]] = wv[i];
   }
+  // the operands of a coefficient's update; those of the first trip (mostly the
+  // only one) are loaded here, so that the transform covers their latency
+  const bool has_prev = !sp.first && (mode == kModeFilter || mode == kModeMoments);
+  const bool has_acc = !sp.first && mode == kModeFilter;
+  const bool has_chi = mom_part && !has_acc;  // shares xa
+  double xc[2][2], xp[2][2], xa[2][2], k2 = 0.0;
+  T xf[2][2];
+#pragma unroll
+  for (int o = 0; o < 2; ++o)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      xc[o][i] = xp[o][i] = xa[o][i] = 0.0;
+      xf[o][i] = T(0);
+    }
+  auto fetch = [&](int j) {
+    if (mode == kModeNoise) return;
+    k2 = ak2[j];
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const size_t e = (size_t)(2 * q + o) * ldx + (i ? ncp : 0) + j;
+        xc[o][i] = Xcur[e];
+        if (fnl) xf[o][i] = fnl[e];
+        if (has_prev) xp[o][i] = Xout[e];
+        if (has_acc) xa[o][i] = acc[e];
+        if (has_chi) xa[o][i] = chi[e];
+      }
+  };
+  if (j0 + tid < j1) fetch(j0 + tid);
   __syncthreads();
   fft_lines_map<T, N, -1, ML, kThreads, kLineFastA<T>>(buf, nc, LD, tw, tid);
 
@@ -315,6 +365,7 @@ __device__ __forceinline__ void contract_body(const ContractArgs& a, int chunk, 
   // (pp, pm) of coefficient j; the increment loads the next trip's pair
   for (int j = j0 + tid, pp = pp_first, pm = pm_first; j < j1;
        j += kThreads, pp = j < j1 ? coef_plus[j] : 0, pm = j < j1 ? coef_minus[j] : 0) {
+    if (j != j0 + tid) fetch(j);
     Cx<T>* bp = &buf[((pp >> 8) - c0) * LD + (pp & 255)];
     Cx<T>* bm = &buf[((pm >> 8) - c0) * LD + (pm & 255)];
     const Cx<T> t = *bp;
@@ -334,7 +385,6 @@ __device__ __forceinline__ void contract_body(const ContractArgs& a, int chunk, 
       f[1][0] = -2.0 * ti;
       f[1][1] = 0.0;
     }
-    const double k2 = ak2[j];
     if (mode == kModeNoise) {
       // c(G) = (1/N) sum_r chi(r) e^{-iG.r} of the two real fields: minus a
       // quarter (G != 0) / half (G = 0) of the unpack
@@ -353,11 +403,11 @@ __device__ __forceinline__ void contract_body(const ContractArgs& a, int chunk, 
 #pragma unroll
     for (int o = 0; o < 2; ++o) {
       const size_t base = (size_t)(2 * q + o) * ldx;
-      const double cr = Xcur[base + j], ci = Xcur[base + ncp + j];
+      const double cr = xc[o][0], ci = xc[o][1];
       double fr = f[o][0], fi = f[o][1];
       if (fnl) {
-        fr += double(fnl[base + j]);
-        fi += double(fnl[base + ncp + j]);
+        fr += double(xf[o][0]);
+        fi += double(xf[o][1]);
       }
       if (!g0) {
         fr -= 2.0 * k2 * cr;
@@ -394,7 +444,7 @@ __device__ __forceinline__ void contract_body(const ContractArgs& a, int chunk, 
           nr = (g0 ? sp.s2 : sp.s1) * fr + sp.p * cr;
           ni = g0 ? fi : sp.s1 * fi + sp.p * ci;
         } else {
-          const double pr = Xout[base + j], pi = Xout[base + ncp + j];
+          const double pr = xp[o][0], pi = xp[o][1];
           nr = (g0 ? sp.s2 : sp.s1) * fr + sp.p * cr - pr;
           ni = g0 ? fi : sp.s1 * fi + sp.p * ci - pi;
         }
@@ -405,15 +455,16 @@ __device__ __forceinline__ void contract_body(const ContractArgs& a, int chunk, 
             acc[base + j] = sp.c0 * cr + sp.ck * nr;
             acc[base + ncp + j] = sp.c0 * ci + sp.ck * ni;
           } else {
-            acc[base + j] += sp.ck * nr;
-            acc[base + ncp + j] += sp.ck * ni;
+            acc[base + j] = xa[o][0] + sp.ck * nr;
+            acc[base + ncp + j] = xa[o][1] + sp.ck * ni;
           }
         }
         if (mom_part) {
           // Gamma dot as coded at calc-chempot-chebyshev.c:725-729:
           // 2 sum re*re + 2 sum im*im - re(0)*re(0)
           const double wr = g0 ? 1.0 : 2.0;
-          const double xr = chi[base + j], xi = chi[base + ncp + j];
+          const double xr = has_chi ? xa[o][0] : chi[base + j];
+          const double xi = has_chi ? xa[o][1] : chi[base + ncp + j];
           dots[0] += wr * xr * nr + 2.0 * xi * ni;
           if (sp.first)
             dots[1] += wr * cr * cr + 2.0 * ci * ci;
