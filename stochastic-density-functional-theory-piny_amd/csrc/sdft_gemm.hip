@@ -17,6 +17,8 @@
 // them with vector loads straight into registers: no LDS staging and no
 // barriers inside the K loop.  Each wave accumulates a 32x32 tile (2x2 MFMA
 // blocks).
+#include <algorithm>
+
 #include "sdft_kb.h"
 
 namespace sdft {
@@ -294,7 +296,8 @@ __global__ __launch_bounds__(256) void k_kb_reduce_force(const double* __restric
 
 int launch_kb_reduce_force(Ctx& c, int prec, int ns, int nsplit, void* fnl) {
   const int K2 = 2 * c.g.ncp, ts = (ns + 31) / 32, tot = ts * (K2 / 64);
-  const size_t lds = (size_t)32 * kb_small_ldy(c.ppad) * (prec == 0 ? 8 : 4);
+  // as many rows as a tile has states: at most kKbFusedTile projections
+  const size_t lds = (size_t)std::min(ns, 32) * kb_small_ldy(c.ppad) * (prec == 0 ? 8 : 4);
   if (prec == 0) {
     auto kern = &k_kb_reduce_force<double>;
     SDFT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),

@@ -263,8 +263,8 @@ __device__ __forceinline__ void kb_force_block(const T* __restrict__ Y, const T*
 }
 
 // The two products of a system too small for a launch each: the split's
-// partials are summed while they are brought into LDS as Y (one tile of 32
-// states, row stride kb_small_ldy), and the force product reads Y from there.
+// partials are summed while they are brought into LDS as Y (one tile of up to
+// 32 states, a row each, row stride kb_small_ldy), and the force product reads Y from there.
 // Workgroup (bx, by): states 32 bx .., columns 64 by .. 64 by + 63 (16 per
 // wave).  Every workgroup sums its tile's partials again: they come from L2
 // (at most kKbFusedPartials of them a tile).

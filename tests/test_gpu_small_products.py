@@ -4,7 +4,8 @@ oracle at the parity tests' bounds (FP64 1e-12, FP32 2e-5) and against the
 general path (another plane tile: its own launches on a second stream), whose
 sums differ in order only (1e-13, 5e-6).  Projector counts below, at and above
 a tile of 32; states of one, part of, one and several tiles; 64 projectors with
-32 states are the largest fused tile, 65 projectors the next."""
+32 states are the largest fused tile, 65 projectors the next; so are 1024 with
+one pair of orbitals, and with two."""
 import numpy as np
 import pytest
 
@@ -20,7 +21,8 @@ def _rel(a, b):
 
 @pytest.mark.parametrize("n,natm,states", [(24, 1, (1, 31)), (24, 16, (2, 32, 65)),
                                            (32, 17, (33,)), (36, 27, (16, 18)),
-                                           (48, 9, (1, 40)), (64, 50, (3, 12))])
+                                           (48, 9, (1, 40)), (64, 50, (3, 12)),
+                                           (24, 200, (1,)), (24, 256, (1, 3))])
 def test_small_products(n, natm, states):
     rng = np.random.default_rng(n + natm)
     g2 = (0.2 * n * 2.0 * np.pi / 10.26) ** 2
