@@ -261,6 +261,10 @@ __global__ __launch_bounds__(kThreads) void k_noise_plane(Cx<double>* __restrict
 // 142.7 -> 118.4 (three launches); 32^3 FP64, 64 orbitals 10.9 -> 9.8; at
 // 64^3, 256 orbitals, where it is near the memory's rate (180 MB), 31.3 -> 30.9
 // in FP32 and 37.9 -> 38.2 in FP64.
+// The chunk's loads are kept as real and imaginary parts: as an array of
+// complex values the FP64 kernel over a batch put them in private memory (64 to
+// 144 bytes a thread; 343 fragments 10.96 ms/step against 10.42, 8 systems of 64
+// orbitals at 64^3 292 us/step against 258).
 template <typename T, int N, bool E>
 __device__ __forceinline__ void contract_body(const ContractArgs& a, int chunk, int q) {
   constexpr int CH = Cfg<N>::CH, LD = Cfg<N>::LD, ML = Cfg<N>::ML;
@@ -314,19 +318,21 @@ __device__ __forceinline__ void contract_body(const ContractArgs& a, int chunk, 
   {
     // all loads of the chunk in flight before the first is stored
     constexpr int ME = (CH * N + kThreads - 1) / kThreads;
-    Cx<T> wv[ME];
+    T wr[ME], wi[ME];
     int slot[ME];
 #pragma unroll
     for (int i = 0; i < ME; ++i) {
       const int e = tid + i * kThreads;
       int dl, ra;
       slot_map<true, 1>(e < nc * N ? e : 0, nc, rnc, dl, ra);
-      wv[i] = Wq[(size_t)ra * ncolp + c0 + dl];
+      const Cx<T> x = Wq[(size_t)ra * ncolp + c0 + dl];
+      wr[i] = x.x;
+      wi[i] = x.y;
       slot[i] = dl * LD + ra;
     }
 #pragma unroll
     for (int i = 0; i < ME; ++i)
-      if (tid + i * kThreads < nc * N) buf[slot[i]] = wv[i];
+      if (tid + i * kThreads < nc * N) buf[slot[i]] = cx(wr[i], wi[i]);
   }
   // the operands of a coefficient's update; those of the first trip (mostly the
   // only one) are loaded here, so that the transform covers their latency
