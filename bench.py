@@ -676,9 +676,12 @@ PLANE_VARIANTS = {0: (0, 256, 0, 0), 1: (1, 256, 0, 0), 2: (0, 256, 0, 1), 3: (1
 
 
 def plane_kernel_name(t, n, variant, pruned):
-    """The plane kernel's instantiation as rocprofv3 names it (variant 0 of a
-    pruned grid up to 128^3 is the stage per wave)."""
-    if variant == 0 and pruned == "true" and n <= 128:
+    """The plane kernel's instantiation beside Kleinman-Bylander products, as
+    rocprofv3 names it: variant 0 of a pruned grid up to 96^3 is the stage per
+    wave, but for 48^3 in FP64 and 64^3 in FP32 (128^3, where it depends on the
+    number of orbitals and on the sphere, is not told apart here)."""
+    if variant == 0 and pruned == "true" and n <= 96 and \
+            (n, t) not in ((48, "double"), (64, "float")):
         return "k_wplane<%s, %d, 0>" % (t, n)
     v, nt, sc, sb = PLANE_VARIANTS[variant if n == 64 else variant & 1]
     return "k_plane<%s, %d, %d, %s, %d, %d, %d>" % (t, n, v, pruned, nt, sc, sb)

@@ -747,18 +747,22 @@ static int apply_step(Block& b, int mode, const double* cur, double* out, const 
   }
   const bool small = table && kb_small_applies(c, b.prec, b.nstate_pad);
   const void* kbx = x32 ? (const void*)b.X32 : (const void*)cur;
-  // Else the KB chain overlaps the FFT kernels.  It follows the previous contract on
-  // that kernel's own stream; the FFT kernels and this step's contract go to
-  // the other one, which then is the context's stream (the two swap roles
-  // every step).  So the chain's projection starts first and has its
-  // workgroups placed before the plane kernel fills the chip: started behind
-  // it (5 us later, the time of an event between streams), it got its slots
-  // only as the plane drained and took 63 us instead of 20 (Si64 FP32).
+  // Else the KB chain overlaps the FFT kernels, on the other stream.  Where it
+  // goes first (kb_chain_first), it follows the previous contract on that
+  // kernel's own stream, and the FFT kernels and this step's contract go to the
+  // other one, which then is the context's stream (the two swap roles): started
+  // behind the plane kernel (5 us later, the time of an event between streams),
+  // its projection got its slots only as the plane drained and took 63 us
+  // instead of 20 (64^3, 256 orbitals, FP32).
   // With profiling on, each kernel's events are recorded on the stream it
   // runs on.
-  if (table && !small) {
+  const bool beside = table && !small;
+  const bool wave = plane_takes_wave(c, b.prec, npairs, beside);
+  if (beside) {
     SDFT_HIP_CHECK(hipEventRecord(c.ev_cur, c.stream));
     SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream_nl, c.ev_cur, 0));
+    const bool split = plane_lds_for(c.g.n, b.prec, c.g.M, 0) > 160 * 1024;
+    if (!kb_chain_first(c.g.n, b.prec, npairs, wave, split)) std::swap(c.stream, c.stream_nl);
     {
       ProfScope ps(c, "kb_project");
       rc = launch_nl_project(c, b.prec, kbx, b.nstate_pad);
@@ -811,9 +815,9 @@ static int apply_step(Block& b, int mode, const double* cur, double* out, const 
     fnl = b.fnl;
   } else {
     ProfScope ps(c, "plane_bc_vpsi");
-    if ((rc = launch_plane(c, b.prec, c.W, npairs, &Wres))) return rc;
+    if ((rc = launch_plane(c, b.prec, c.W, npairs, wave, &Wres))) return rc;
   }
-  if (table && !small) SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream, c.ev_nl, 0));
+  if (beside) SDFT_HIP_CHECK(hipStreamWaitEvent(c.stream, c.ev_nl, 0));
   {
     ProfScope ps(c, "contract_a");
     if ((rc = launch_contract(c, b.prec, mode, Wres, npairs, cur, out, b.acc, fnl, b.chi, sp,

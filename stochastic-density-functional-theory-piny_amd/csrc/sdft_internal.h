@@ -102,9 +102,12 @@ constexpr size_t kKeepBytes = size_t(256) << 20;
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
-  // the KB GEMM chain of a step runs on stream_nl, concurrently with the
-  // expand / plane kernels; ev_cur orders it after the previous step, ev_nl
-  // orders the contract kernel after it
+  // the KB product chain of a step runs on one of the two streams, the expand,
+  // plane and contract kernels on the other; ev_cur orders the streams after
+  // the previous step, ev_nl the contract after the chain.  Where the chain is
+  // put ahead (kb_chain_first) it takes `stream`, and the two handles swap: read
+  // c.stream again after every step; what it names then is behind all of the
+  // step's work.
   hipStream_t stream_nl = nullptr;
   hipEvent_t ev_cur = nullptr;
   hipEvent_t ev_nl = nullptr;
@@ -362,7 +365,8 @@ int launch_expand(Ctx& c, int prec, const double* X, int npairs, void* W);
 // *Wout receives the buffer holding the result: W itself, or the context's
 // second buffer W2 when the plane runs in the split form (M x (n+1) plane
 // buffer above the LDS size)
-int launch_plane(Ctx& c, int prec, void* W, int npairs, void** Wout);
+// wave: the stage per wave (plane_takes_wave)
+int launch_plane(Ctx& c, int prec, void* W, int npairs, bool wave, void** Wout);
 // Plane-kernel variants offered at grid size n (b-line tile, threads per
 // workgroup, radix schedules): 6 at n = 64, 2 elsewhere.
 inline int plane_variant_count(int n) { return n == 64 ? 6 : 2; }
@@ -421,6 +425,41 @@ size_t wplane_lds_for(int n, int prec, int M);
 inline bool wplane_applies(const Ctx& c, int prec, int mode) {
   return plane_prunable(c.g.K, c.g.n) && wplane_lds_for(c.g.n, prec, c.g.M) > 0 &&
          !(mode != 0 && prec == 1 && c.g.n > 48);
+}
+// Beside a KB chain on the other stream the two plane stages compete with it for
+// the CUs, and the stage that is faster alone need not give the faster step.
+// us per filter step, stage per wave / workgroup-wide, the chain ahead of both
+// (states: us):
+//   FP64  48  128: 90 / 80   256: 142 / 138   512: 250 / 245
+//         64  128: 100 / 119   256: 177 / 215   640: 399 / 503
+//         96  8: 73 / 94   64: 263 / 290       128  1: 684 / 546   8: 844 / 574
+//                                               32: 880 / 756   64: 1284 / 1434
+//   FP32  48  256: 93 / 103   700: 203 / 232    64  192: 95 / 92   256: 116 / 115
+//         96  8: 58 / 57   64: 141 / 153       128  8: 346 / 276   32: 374 / 358
+//                                               64: 672 / 685
+// At 128 a workgroup of the stage per wave fills the registers of a CU, so it
+// waits for one that no workgroup of the chain is on; with few pairs (up to one
+// 32-state tile of the products) the chain is most of the step.
+bool wave_beside_kb(int n, int prec, int npairs);
+// Whether the chain is queued ahead of the plane stage, on the previous
+// contract's own stream, or behind it on the other stream.  Ahead, its
+// projection has its workgroups placed before the plane kernel fills the chip;
+// the workgroup-wide stage then starts late, which costs more the more of it
+// there is: chain ahead / behind, us per filter step
+//   FP64  48  300: 158 / 166   400: 200 / 202   450: 222 / 218   512: 245 / 240
+//        128  8: 572 / 640   24: 673 / 689   28: 714 / 693   32: 756 / 724
+//   FP32  64  300: 132 / 137   320: 139 / 138   384: 161 / 156   640: 253 / 247
+// (kKbBehindBytes of pair grids).  At 192, and in the split form, it goes behind:
+//   FP64 192  2: 1079 / 1020   8: 1440 / 1471   32: 2998 / 2960
+//   FP32 192  2: 506 / 602     8: 681 / 637     32: 1486 / 1411
+// The stage per wave keeps the chain ahead at every size measured (64, FP64,
+// 256: 177 / 201; 48, FP32, 256: 93 / 107).
+constexpr size_t kKbBehindBytes = size_t(320) << 20;
+bool kb_chain_first(int n, int prec, int npairs, bool wave, bool split);
+// the stage of a whole plane pass (variant 0 only): per wave, or workgroup-wide
+inline bool plane_takes_wave(const Ctx& c, int prec, int npairs, bool beside_kb) {
+  return c.plane_variant == 0 && wplane_applies(c, prec, 0) &&
+         (!beside_kb || wave_beside_kb(c.g.n, prec, npairs));
 }
 // Small systems: the KB projection in the plane stage's launch, the reduction
 // and the force product behind it on the same stream.  Against the chain on a

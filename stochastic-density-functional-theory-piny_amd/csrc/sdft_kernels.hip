@@ -888,7 +888,8 @@ static int plane_launch(Ctx& c, const PlaneArgs& a, size_t lds, int npairs) {
 // Plane-kernel variants (the tuner's plane tile): b-line tile V, threads per
 // workgroup NT and the radix schedules of the c- and b-lines (SC, SB).
 // Variant 0 is the wave-private stage (sdft_plane_wave.h) where it applies,
-// and the one listed here elsewhere (spheres beyond n/4, n = 192).  At
+// and the one listed here elsewhere (spheres beyond n/4, n = 192, planes that
+// do not fit LDS, and beside a KB chain as wave_beside_kb says).  At
 // n = 64 every thread of a pass has a butterfly when (lines x butterflies
 // per line) reaches NT: with radix-4 b-lines (SB = 1) a 256-thread FP64
 // workgroup fills its threads from a 16-line b tile, and 512-thread ones keep
@@ -955,8 +956,8 @@ static int plane_impl(Ctx& c, void* W, int npairs, void** Wout) {
   return 0;
 }
 
-int launch_plane(Ctx& c, int prec, void* W, int npairs, void** Wout) {
-  if (c.plane_variant == 0 && wplane_applies(c, prec, 0)) {
+int launch_plane(Ctx& c, int prec, void* W, int npairs, bool wave, void** Wout) {
+  if (wave) {
     *Wout = W;
     return launch_wplane(c, prec, make_plane_args(c, prec, W), npairs, 0);
   }

@@ -144,6 +144,17 @@ static int wplane_project_t(Ctx& c, const PlaneArgs& a, const KbProjectArgs& p, 
   }
 }
 
+bool wave_beside_kb(int n, int prec, int npairs) {
+  if (n == 128) return npairs > 16;
+  return prec == 0 ? n != 48 : n != 64;
+}
+
+bool kb_chain_first(int n, int prec, int npairs, bool wave, bool split) {
+  const size_t bytes = (prec == 0 ? sizeof(Cx<double>) : sizeof(Cx<float>)) * (size_t)npairs *
+                       (size_t)n * n * n;
+  return wave || (n < 192 && !split && bytes < kKbBehindBytes);
+}
+
 bool kb_small_applies(const Ctx& c, int prec, int ns) {
   const double force = 2.0 * ((ns + 31) / 32 * 32) * c.ppad * 2.0 * c.g.ncp;
   return c.g.n <= 64 && c.plane_variant == 0 && wplane_applies(c, prec, 0) &&
