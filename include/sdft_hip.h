@@ -57,7 +57,15 @@ typedef struct sdft_grid_desc {
 } sdft_grid_desc;
 
 /* Create a context on the current HIP device.  Replaces the FFTW plan and map
- * set-up of fft_create_package.c:1627-1689 for the filter's grid. */
+ * set-up of fft_create_package.c:1627-1689 for the filter's grid.
+ * Besides its tables, potential and projectors a context keeps work memory
+ * from one call to the next, as large as its largest call needed: the
+ * transform and projection buffers without a bound, and for calls on host
+ * arrays the orbital block, its moment partials and their scratch, at most 256
+ * MiB each (a call that needs more allocates and frees its own), device
+ * staging of 64 MiB (or one state) and 768 KiB of pinned host memory.
+ * sdft_hip_finalize releases all of it; a program with hundreds of contexts
+ * that are done with such calls may want to finalize them. */
 int sdft_hip_init(const sdft_grid_desc *desc, sdft_ctx **out);
 int sdft_hip_finalize(sdft_ctx *ctx);
 const char *sdft_hip_last_error(void);

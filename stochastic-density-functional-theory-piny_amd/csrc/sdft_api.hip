@@ -665,6 +665,10 @@ struct CallBlock {
     if (own && b) {
       block_free(*b);
       delete b;
+    } else if (b && b->mom_part_bytes > kKeepBytes) {  // grows with the degree
+      (void)hipFree(b->mom_part);
+      b->mom_part = nullptr;
+      b->mom_part_bytes = 0;
     }
   }
 };

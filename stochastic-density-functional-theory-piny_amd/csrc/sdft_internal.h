@@ -94,9 +94,9 @@ struct RsKB;
 struct Block;
 
 // Device memory that a context keeps between calls for the calls' own use
-// (orbital blocks of calls on host arrays, partial sums): per buffer at most
-// this much; a call that needs more allocates for itself and frees at its
-// end.  Everything is released with the context.
+// (the orbital block of calls on host arrays, its moment partials, the calls'
+// scratch): each at most this much; a call that needs more allocates for itself
+// and frees at its end.  Everything is released with the context.
 constexpr size_t kKeepBytes = size_t(256) << 20;
 
 struct Ctx {
