@@ -324,7 +324,9 @@ int sdft_hip_batch_config(sdft_batch *bat, int split, int overlap, int plane_til
  * variant, target, fused expand.  Returns the number of candidates (2 x 2 x
  * 2 per variant pair: 24 at n = 64, 8 elsewhere; half without the fused
  * form).  sdft_hip_set_config sets the three knobs by hand (variant in
- * [0, 6) at n = 64, [0, 2) elsewhere). */
+ * [0, 6) at n = 64, [0, 2) elsewhere).  Small systems do not use the target
+ * with variant 0; where that is the fastest, the target kept is that of the
+ * fastest candidate that used it. */
 int sdft_hip_tune(sdft_ctx *ctx, int nstate, int prec, int steps, int *config_out, int max_cand,
                   double *cand_ms);
 int sdft_hip_set_config(sdft_ctx *ctx, int plane_tile, int kb_wg_target, int fused_expand);

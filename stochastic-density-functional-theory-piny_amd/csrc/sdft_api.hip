@@ -1375,6 +1375,14 @@ int sdft_hip_tune(sdft_ctx* h, int nstate, int prec, int steps, int* config_out,
   int best_pv = pv0, best_kt = kt0, ncand = 0;
   bool best_fu = fu0;
   double best = 1e300;
+  // small systems' products ride in the plane stage's launch and leave the
+  // target alone: where such a candidate is the fastest, the target is that of
+  // the fastest one that used it (noise would choose it else, for the energies,
+  // forces and larger blocks that do use it)
+  const bool table = c.nproj > 0 && !rs_active(c);
+  int kt_used = kt0;
+  bool best_used = true;
+  double best_of_used = 1e300;
   const int L = steps + 4;
   double* bufs[2] = {b.X0, b.X1};
   auto step_params = [](int k) {
@@ -1393,6 +1401,7 @@ int sdft_hip_tune(sdft_ctx* h, int nstate, int prec, int steps, int* config_out,
         c.plane_variant = pv;
         c.kb_wg_target = targets[ti];
         c.fuse_expand = fu != 0;
+        const bool used = !table || !kb_small_applies(c, prec, b.nstate_pad);
         for (int k = 1; k <= 2 && !rc; ++k)  // warm-up: the first two steps
           rc = apply_step(b, kModeFilter, bufs[(k - 1) & 1], bufs[k & 1], step_params(k),
                           nullptr, fuse_flags(c, k, L));
@@ -1420,8 +1429,14 @@ int sdft_hip_tune(sdft_ctx* h, int nstate, int prec, int steps, int* config_out,
           best_pv = pv;
           best_kt = targets[ti];
           best_fu = fu != 0;
+          best_used = used;
+        }
+        if (used && per < best_of_used) {
+          best_of_used = per;
+          kt_used = targets[ti];
         }
       }
+  if (!best_used) best_kt = kt_used;
   c.profiling = prof;
   if (t0) (void)hipEventDestroy(t0);
   if (t1) (void)hipEventDestroy(t1);
