@@ -1282,13 +1282,15 @@ int sdft_hip_nl_forces(sdft_ctx* h, int nstate, const double* re, const double* 
       set_error("projector atom index out of range");
       return SDFT_EINVAL;
     }
+  const int ncp = c.g.ncp;
+  // ends of queued copies: they outlive cb, whose end waits for the stream
+  std::vector<double> gint((size_t)3 * ncp, 0.0), hs((size_t)3 * P);
   CallBlock cb(c);
   CallArena ar(c);
   int rc = cb.get(nstate, 0);
   if (rc) return rc;
   Block& b = *cb.b;
-  const int ns = b.nstate_pad, ncp = c.g.ncp;
-  std::vector<double> gint((size_t)3 * ncp, 0.0);
+  const int ns = b.nstate_pad;
   for (int j = 0; j < c.g.ncoef; ++j)
     for (int d = 0; d < 3; ++d) gint[(size_t)d * ncp + j] = gvec[(size_t)c.g.perm[j] * 3 + d];
   int per = 0;
@@ -1301,7 +1303,6 @@ int sdft_hip_nl_forces(sdft_ctx* h, int nstate, const double* re, const double* 
   double *dg = ar.take<double>(ng), *Ad = ar.take<double>(nad), *Zd = ar.take<double>(nzd),
          *part = ar.take<double>(npt), *S = ar.take<double>(nS);
   if ((rc = block_put(b, b.X0, re, im))) return rc;
-  std::vector<double> hs((size_t)3 * P);
   hipError_t e = hipMemcpyAsync(dg, gint.data(), sizeof(double) * ng, hipMemcpyHostToDevice,
                                 c.stream);
   // zero padding rows
@@ -1974,6 +1975,7 @@ int sdft_hip_ks_potential(sdft_ctx* h, const double* rho, int layout, const doub
   SDFT_HIP_CHECK(hipMemcpyAsync(c.ks_io, rho, sizeof(double) * N, hipMemcpyHostToDevice, s));
   if ((rc = launch_ks_field(s, c.ks_io, layout, n, N, volume, c.ks_field, c.ks_rho))) return rc;
   if ((rc = ensure_W(dc, w_bytes(dc, 1, 0)))) return rc;
+  std::vector<double> part;  // end of a queued copy: outlives cb
   CallBlock cb(dc);
   if ((rc = cb.get(1, 0))) return rc;
   Block& b = *cb.b;
@@ -1998,7 +2000,6 @@ int sdft_hip_ks_potential(sdft_ctx* h, const double* rho, int layout, const doub
   // + LDA exchange-correlation -> the context's v_KS
   if (!rc)
     rc = launch_ks_xc(s, c.ks_vhe, c.ks_rho, N, xc, c.vks64, c.vks32, c.ks_part + 2 * nb1, &nb2);
-  std::vector<double> part;
   if (!rc) {
     part.resize(2 * (size_t)(nb1 + nb2));
     SDFT_HIP_CHECK(hipMemcpyAsync(part.data(), c.ks_part, sizeof(double) * part.size(),
