@@ -165,6 +165,12 @@ bool kb_small_fused(const Ctx& c, int ns) {
   return c.ppad * std::min(ns, 32) <= kKbFusedTile;
 }
 
+// waves of a workgroup, which share a tile of the projection
+static int wplane_waves(int n) {
+  SDFT_WPLANE_SWITCH(n, return WaveCfg<NN>::NW);
+  return SDFT_EINVAL_CODE;
+}
+
 int launch_plane_project(Ctx& c, int prec, void* W, int npairs, const void* X, int ns,
                          int* nsplit) {
   const int P = c.nproj, K = 2 * c.g.ncp, nsteps = K / 32;
@@ -177,7 +183,8 @@ int launch_plane_project(Ctx& c, int prec, void* W, int npairs, const void* X, i
   p.tp = (P + 31) / 32;
   p.ts = (ns + 31) / 32;
   const int tiles = p.tp * p.ts;
-  const int waves = c.g.n <= 32 ? 1 : c.g.n == 36 ? 2 : 3;  // WaveCfg::NW
+  const int waves = wplane_waves(c.g.n);
+  if (waves < 0) return waves;
   const bool fused = kb_small_fused(c, ns);
   int s = (nsteps + waves - 1) / waves;  // one step of the sum per wave
   s = std::min(s, ((fused ? 256 : 128) + tiles - 1) / tiles);
