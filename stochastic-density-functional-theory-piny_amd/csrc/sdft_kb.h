@@ -92,6 +92,13 @@ __device__ __forceinline__ void kb_project_tile(const TA* __restrict__ A,
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = TI(0);
+  // Without AHEAD a split is many steps long (few splits, so that there are few
+  // partials to read again), and each step's sums go to FP64 sums of their own:
+  // one chain over the split rounded worse than the short chains of many splits
+  // (H psi of 8 orbitals at 64^3, error of its norm: FP32 3.8e-8, with these sums
+  // 2.4e-8, short chains 2.8e-8; FP64 8.9e-17, 6.7e-17, 7.0e-17).
+  constexpr int NS = AHEAD ? 1 : 2;
+  double sum[NS][NS][2 * NS] = {};
   const int step0 = bz * ksteps_per_split;
   const int nsteps_total = K / KS;
   const int step1 = min(nsteps_total, step0 + ksteps_per_split);
@@ -148,6 +155,15 @@ __device__ __forceinline__ void kb_project_tile(const TA* __restrict__ A,
     for (; st < step1; st += NWV) {
       load_raw(st, ra0, rb0);
       mma_raw(ra0, rb0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            sum[i][j][r] += double(acc[i][j][r]);
+            acc[i][j][r] = TI(0);
+          }
     }
   }
   // sum the waves' tiles
@@ -159,7 +175,10 @@ __device__ __forceinline__ void kb_project_tile(const TA* __restrict__ A,
       for (int r = 0; r < 4; ++r) {
         const int row = 16 * i + Mfma<TI>::row(lane, r);
         const int col = 16 * j + r16;
-        red[wave * 1024 + row * 32 + col] = double(acc[i][j][r]);
+        if constexpr (AHEAD)
+          red[wave * 1024 + row * 32 + col] = double(acc[i][j][r]);
+        else
+          red[wave * 1024 + row * 32 + col] = sum[i][j][r];
       }
   __syncthreads();
   double* zp = zpart + (size_t)bz * P * ns;
