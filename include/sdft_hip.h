@@ -315,7 +315,8 @@ int sdft_hip_batch_config(sdft_batch *bat, int split, int overlap, int plane_til
  * expand (0: an expand kernel per step, 1: the contract kernel writes the
  * next step's a-expansion; offered only when every sphere column is one ka
  * interval) -- and keeps the fastest for this context.  Plane variants: 0
- * the base b-line tile, 1 twice as wide (where it fits LDS); at n = 64 also
+ * a wave per group of lines or the base b-line tile, by what was measured for
+ * the size, form and block, 1 twice as wide (where it fits LDS); at n = 64 also
  * 2 radix-4 b-lines (4x4x4 instead of 8x8) on the base tile, 3-5 512-thread
  * workgroups with radix-4 c-lines (3: wide tile, radix-8 b-lines; 4: wide
  * tile, radix-4 b-lines; 5: base tile, radix-4 b-lines).  config_out

@@ -409,13 +409,14 @@ size_t plane_lds_for(int n, int prec, int M, int variant);
 // |k| < n/4 on every axis
 inline bool plane_prunable(int K, int n) { return 4 * K < n; }
 // wave-private plane stage (sdft_wplane.hip), spheres inside |k| < n/4: its
-// dynamic LDS (0: grid size not built), its launch (mode 0 fused, 1 / 3 to the
+// dynamic LDS (0: not built, or over 160 KB), its launch (mode 0 fused, 1 / 3 to the
 // grid a.field, 2 from it) and its launch over the fragments of a batch
 size_t wplane_lds_for(int n, int prec, int M);
 // Whether a stage of `mode` takes it: wherever it is built, fits LDS and was
-// measured faster.  That is the whole stage at every size (sdft_plane_wave.h),
-// and of the halves to and from the grid (us, mode 2 / mode 1, this stage
-// against the workgroup-wide one, 256 orbitals at 48 and 64, 64 at 128)
+// measured faster.  That is the whole stage at every size (sdft_plane_wave.h;
+// beside KB products plane_takes_wave decides), and of the halves to and from the
+// grid (us, mode 2 / mode 1, this stage against the workgroup-wide one, 256
+// orbitals at 48 and 64, 64 at 128)
 //   FP64  48: 44.5 / 42.2 against 49.4 / 51.0    96: 146 / 118 against 167 / 121
 //         64: 126 / 102 against 126 / 119       128: 311 / 267 against 330 / 277
 //   FP32  48: 27.0 / 25.2 against 34.6 / 32.3    96: 68.5 / 56.6 against 59.0 / 55.0
